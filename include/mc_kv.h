@@ -223,7 +223,9 @@ mc_status_t mc_kv_attention_decode_batch(const uint16_t* d_q_rows,
  * causal attention of T query rows (absolute positions *d_base_pos + t) over
  * pool positions 0..*d_base_pos + t gathered through the page table.
  * S_kv in 1..8 key splits; S_kv > 1 needs d_partials of
- * T*16*S_kv*130 floats and runs the split merge. Writes d_out [T][2048]. */
+ * T*16*S_kv*130 floats and runs the split merge. For short chunks it is the
+ * most splits: a launch whose rows fill the GPU by themselves uses fewer.
+ * Writes d_out [T][2048]. */
 mc_status_t mc_kv_attention_prefill(const uint16_t* d_q_rows, uint32_t tokens,
                                     const uint32_t* d_base_pos, uint32_t layer,
                                     const uint32_t* d_page_table,
@@ -336,7 +338,8 @@ mc_status_t mc_debug_batch_group_stats(mc_batch_group_t group, uint64_t* steps,
 int mc_debug_batch_breakdown_collect(mc_batch_group_t group, double* out_ms, int n);
 
 /* Prefill workgroup shape: 0 = 32 query rows on 8 waves, 1 = 16 rows on 4
- * waves, 2 = 16 rows on two 4-wave halves taking alternate key steps,
+ * waves, 2 = 16 rows on two 4-wave halves taking alternate key steps, 3 and
+ * 4 = 8 and 4 rows on four key sets taking alternate 32-key blocks,
  * 0xFFFFFFFF = chosen per launch (default). All compute the same softmax;
  * shapes differ in tile boundaries (key splits) and summation order, within
  * the attention tolerance. The previous value is stored to *previous when

@@ -44,6 +44,7 @@
 // and differ only in rounding.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 
@@ -63,10 +64,16 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 //            P.V; one workgroup per CU (107 KB LDS);
 //   kRows16: 256 threads, 4 waves, 16 q rows, two LDS buffers; two per CU;
 //   kHalves: 512 threads, 16 q rows, two 4-wave halves on alternate key steps
-//            (two LDS buffers each) merged in LDS at the end; one per CU.
-constexpr uint32_t kRows32 = 0u, kRows16 = 1u, kHalves16 = 2u;
+//            (two LDS buffers each) merged in LDS at the end; one per CU;
+// and, outside this template, the key-set shapes (prefill_sets_kernel):
+//   kSets8:  1024 threads, 8 q rows, four key sets; one per CU;
+//   kSets4:  512 threads, 4 q rows, four key sets.
+constexpr uint32_t kRows32 = 0u, kRows16 = 1u, kHalves16 = 2u, kSets8 = 3u, kSets4 = 4u;
 // 32-row workgroup count (2 per CU) below which the 16-row shapes are used.
 constexpr uint32_t kSmallBelow = 512u;
+// Rows up to which a launch without / with key splits runs on the key-set
+// workgroups (the reasons stand at the choice below).
+constexpr uint32_t kSetsRows = 1024u, kSetsSplitRows = 384u;
 // Polls of a per-half barrier before it gives up (s_sleep 1 = 64 clocks each,
 // about 2^22 * 64 / 2.4 GHz = 0.1 s): far beyond any legal wait, so it only
 // ends a wait that can never complete. A timed-out wait is counted in
@@ -634,29 +641,301 @@ __global__ void __launch_bounds__(PfShape<SH>::kThreads)
     }
 }
 
-// grid = T*16 (block = (t, qh)), block = 128 (thread = dim).
-__global__ void __launch_bounds__(128) prefill_merge_kernel(
-    const float* __restrict__ partials, uint32_t S, uint32_t T,
-    uint16_t* __restrict__ out) {
-    const uint32_t bh = blockIdx.x;
-    const uint32_t t = bh >> 4;
-    if (t >= T) return;
-    const uint32_t d = threadIdx.x;
+// ---- short chunks: key-set workgroups ----
+// With a few hundred rows a workgroup per 16 rows leaves most CUs idle and
+// each one's time is the chain of its key steps. Here a workgroup takes 2 * CG
+// rows (CG waves of 16 query columns: 2 rows x 8 heads) and kSets key sets of
+// CG waves: set k runs the 32-key blocks b0 + k, b0 + k + kSets, ..., so an
+// iteration covers 128 keys and the chain is a quarter as long; the sets'
+// softmax states are folded in LDS at the end (M = max over the sets, factors
+// exp2((m - M) c)). K/V rows go straight to LDS (global -> LDS loads of 4
+// rows x 256 bytes, two stages per set), unpadded, the 16-byte chunk c of row
+// r at slot c ^ 2 (r mod 8): conflict-free for the K operand reads and the
+// transposing V reads (SQ_LDS_BANK_CONFLICT 0). Rows past key_end repeat the
+// last row (their scores are masked).
+// What bounds it: an iteration's phases (K reads, S, softmax, V reads, P.V)
+// run in step in all waves between two barriers, 1.45 us per 128 keys where
+// the MFMAs alone take 0.45. Against the two-half 16-row shape (us per layer):
+// 64 rows 11.2 -> 5.9, 201 13.0 -> 7.1, 512 18.4 -> 11.0, 1024 27.5 -> 19.5
+// at base 0; 300 rows at base 8000 with 8 splits asked for 56.7 -> 43.1.
+constexpr uint32_t kSets = 4u;       // key sets per workgroup
+constexpr uint32_t kSetBlock = 32u;  // keys per set and iteration
+
+// Waits for all of this wave's global -> LDS loads and its LDS reads (the
+// compiler does not track the LDS side of such loads).
+__device__ __forceinline__ void wait_lds_loads() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+}
+
+// PAGED: a 32-key block lies in one page (P >= 32), whose id is read through
+// the scalar path an iteration ahead.
+template <bool PAGED, uint32_t CG>
+__global__ void __launch_bounds__(64u * CG * kSets)
+    __attribute__((amdgpu_waves_per_eu(CG == 4u ? 4 : 2))) prefill_sets_kernel(
+        const uint16_t* __restrict__ q_rows, uint32_t T, const uint32_t* __restrict__ d_base_pos,
+        uint32_t layer, const uint32_t* __restrict__ pt, const uint16_t* __restrict__ pool,
+        DevLayout ly, uint16_t* __restrict__ out, float* __restrict__ partials, uint32_t S) {
+    constexpr uint32_t kQRows = 2u * CG, KB = kSetBlock;
+    constexpr uint32_t LPW = KB / 2u / CG;        // loads per wave and block (K rows, V rows)
+    constexpr uint32_t kStage = 2u * KB * kD;     // elements of one set's stage
+    constexpr uint32_t kFold = CG * kSets * 64u * 64u;  // all waves' acc, in elements
+    constexpr uint32_t kRing = 2u * kSets * kStage;
+    __shared__ __align__(1024) uint16_t ring[kRing > kFold ? kRing : kFold];
+    __shared__ float2 sml[CG * kSets][16];
+    const uint32_t base_pos = *d_base_pos;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t cg = wave % CG, set = wave / CG;
+    const uint32_t col = lane & 15u, grp = lane >> 4;
+
+    const uint32_t ntq = (T + kQRows - 1u) / kQRows, job = blockIdx.x;
+    const uint32_t s = job % S, kvh = (job / S) % kHkv;
+    const uint32_t tb = (ntq - 1u - job / (S * kHkv)) * kQRows;  // heavy tiles first
+    const uint32_t key_end = base_pos + tb + min(kQRows - 1u, T - 1u - tb);  // last key
+    const uint32_t last = key_end / KB;
+    const uint32_t per = (last + S) / S;  // blocks per split, ceil((last + 1) / S)
+    const uint32_t b0 = s * per, b1 = min(b0 + per - 1u, last);
+
+    auto swz = [](uint32_t r) { return (r & 7u) << 1; };
+    // Lane offset (elements) of load i within its block's slots: K rows 4j..4j+3
+    // or V rows, j = (i * CG + cg) mod 8.
+    uint32_t loff[LPW];
+#pragma unroll
+    for (uint32_t i = 0; i < LPW; ++i) {
+        const uint32_t idx = i * CG + cg, key = 4u * (idx & 7u) + (lane >> 4);
+        loff[i] = key * kSlotElems + (idx >> 3) * 256u + kvh * kD +
+                  8u * ((lane & 15u) ^ swz(key));
+    }
+    uint32_t page = 0u;
+    auto fetch_page = [&](uint32_t b) {
+        if constexpr (PAGED)
+            page = clamp_page(ly, ((const __attribute__((address_space(4))) uint32_t*)(
+                                      pt))[__builtin_amdgcn_readfirstlane(table_index(ly, b * KB))]);
+    };
+    auto load = [&](uint32_t b, uint32_t buf) {
+        uint16_t* l = ring + (buf * kSets + set) * kStage;
+        auto to_lds = [&](const uint16_t* g, uint32_t i) {
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void*)g,
+                (__attribute__((address_space(3))) void*)(l + (i * CG + cg) * 512u), 16, 0, 0);
+        };
+        if (PAGED && b * KB + KB - 1u <= key_end) {  // wave-uniform: every row exists
+            const uint16_t* g = pool + token_base(ly, layer, page, (b * KB) & ly.pmask);
+#pragma unroll
+            for (uint32_t i = 0; i < LPW; ++i) to_lds(g + loff[i], i);
+            return;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < LPW; ++i) {
+            const uint32_t key = 4u * ((i * CG + cg) & 7u) + (lane >> 4);
+            const uint32_t pos = min(b * KB + key, key_end);
+            const uint32_t pg = clamp_page(ly, pt[table_index(ly, pos)]);
+            to_lds(pool + token_base(ly, layer, pg, pos & ly.pmask) + (loff[i] - key * kSlotElems),
+                   i);
+        }
+    };
+    const uint32_t bf = b0 + set;  // this set's first block
+    if (bf <= b1) {
+        fetch_page(bf);
+        load(bf, 0u);
+        if (bf + kSets <= b1) fetch_page(bf + kSets);
+    }
+    // Query column: head col % 8 of row 2 cg + col / 8.
+    const uint32_t row = tb + 2u * cg + (col >> 3);
+    bf16x8 qb[4];
+    {
+        const bool ok = row < T;
+        const uint16_t* q = q_rows + (size_t)(ok ? row : tb) * kRow +
+                            (kvh * kGroup + (col & 7u)) * kD + 8u * grp;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const uint4 v = *reinterpret_cast<const uint4*>(q + 32u * m);
+            qb[m] = as_bf16x8(ok ? v : make_uint4(0u, 0u, 0u, 0u));
+        }
+    }
+    // Softmax state and fast path as in prefill_job.
+    constexpr float kC = kScoreScale * 1.4426950408889634f;
+    constexpr float kMoveSlack = 8.f / kC, kSumCap = 256.f;
+    float m_run = -INFINITY, l_run = 0.f, thr = -INFINITY, nmc = 0.f;
+    f32x4 acc[8];
+#pragma unroll
+    for (int db = 0; db < 8; ++db) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // LDS offsets of the K operand slices and of the V column blocks
+    uint32_t ko[4], vo[8];
+#pragma unroll
+    for (uint32_t m = 0; m < 4u; ++m) ko[m] = col * kD + 8u * ((4u * m + grp) ^ swz(col));
+    const uint32_t vrow = 4u * grp + (col >> 2);
+#pragma unroll
+    for (uint32_t db = 0; db < 8u; ++db)
+        vo[db] = KB * kD + vrow * kD + 8u * ((2u * db + ((col & 3u) >> 1)) ^ swz(vrow)) +
+                 4u * (col & 1u);
+
+    const uint32_t nit = b0 <= b1 ? (b1 - b0) / kSets + 1u : 0u;  // same for all waves
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    for (uint32_t it = 0; it < nit; ++it) {
+        const uint32_t b = bf + it * kSets;
+        wait_lds_loads();
+        __builtin_amdgcn_s_barrier();  // block b is in LDS, block b - kSets is done with
+        if (b + kSets <= b1) {
+            load(b + kSets, (it + 1u) & 1u);
+            if (b + 2u * kSets <= b1) fetch_page(b + 2u * kSets);
+        }
+        if (b > b1) continue;  // wave-uniform; only in the last iteration
+        const uint16_t* st = ring + ((it & 1u) * kSets + set) * kStage;
+        f32x4 sacc[2];
+        {
+            bf16x8 ka[8];
+#pragma unroll
+            for (int o = 0; o < 8; ++o)
+                ka[o] = as_bf16x8(
+                    *reinterpret_cast<const uint4*>(st + (o & 1) * 16u * kD + ko[o >> 1]));
+#pragma unroll
+            for (int o = 0; o < 8; ++o)
+                sacc[o & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    ka[o], qb[o >> 1], o < 2 ? f32x4{0.f, 0.f, 0.f, 0.f} : sacc[o & 1], 0, 0, 0);
+        }
+        if (b * KB + KB - 1u > base_pos + tb) {  // masked keys possible
+            const uint32_t pos0 = b * KB + 4u * grp;
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (pos0 + 16u * kb + (uint32_t)j > base_pos + row) sacc[kb][j] = -INFINITY;
+        }
+        bf16x8 pb;
+        auto probs = [&] {
+            float ls = 0.f;
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float p = __builtin_amdgcn_exp2f(fmaf(sacc[kb][j], kC, nmc));
+                    ls += p;
+                    pb[4 * kb + j] = (__bf16)p;
+                }
+            return ls;
+        };
+        bool done = false;
+        if (__builtin_amdgcn_ballot_w64(m_run == -INFINITY) == 0u) {
+            const float ls = probs();
+            if (__builtin_amdgcn_ballot_w64(ls > kSumCap) == 0u) {
+                l_run += ls;
+                done = true;
+            }
+        }
+        if (!done) {
+            float tm = fmaxf(fmaxf(fmaxf(sacc[0][0], sacc[0][1]), fmaxf(sacc[0][2], sacc[0][3])),
+                             fmaxf(fmaxf(sacc[1][0], sacc[1][1]), fmaxf(sacc[1][2], sacc[1][3])));
+            tm = max_across_groups(tm);
+            float ren = 1.f;
+            if (tm > thr) {
+                ren = __builtin_amdgcn_exp2f((m_run - tm) * kC);
+                l_run *= ren;
+                m_run = tm;
+                thr = tm + kMoveSlack;
+                nmc = -tm * kC;
+            }
+            l_run += probs();
+            if (__builtin_amdgcn_ballot_w64(ren != 1.f) != 0u) {
+#pragma unroll
+                for (int db = 0; db < 8; ++db) acc[db] = acc[db] * ren;
+            }
+        }
+        // contraction index i of lane group grp <-> key 16 (i / 4) + 4 grp + i % 4
+#pragma unroll
+        for (int db = 0; db < 8; ++db) {
+            const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+                (__attribute__((address_space(3))) bf16x4*)(st + vo[db]));
+            const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+                (__attribute__((address_space(3))) bf16x4*)(st + vo[db] + 16u * kD));
+            acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), pb, acc[db], 0, 0, 0);
+        }
+    }
+    l_run += __shfl_xor(l_run, 16);
+    l_run += __shfl_xor(l_run, 32);
+    // Fold: every wave leaves its state in LDS; wave (cg, set) finishes the
+    // two 16-dim blocks 2 set, 2 set + 1 of its columns.
+    __syncthreads();
+    f32x4* sa = reinterpret_cast<f32x4*>(ring);
+#pragma unroll
+    for (int db = 0; db < 8; ++db) sa[(wave * 8u + db) * 64u + lane] = acc[db];
+    if (grp == 0u) sml[wave][col] = make_float2(m_run, l_run);
+    __syncthreads();
+    float M = -INFINITY, L = 0.f;
+    float2 ml[kSets];
+#pragma unroll
+    for (uint32_t k = 0; k < kSets; ++k) {
+        ml[k] = sml[k * CG + cg][col];
+        M = fmaxf(M, ml[k].x);
+    }
+    f32x4 o[2] = {};
+#pragma unroll
+    for (uint32_t k = 0; k < kSets; ++k) {
+        const float f = ml[k].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((ml[k].x - M) * kC);
+        L += ml[k].y * f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) o[i] += sa[((k * CG + cg) * 8u + 2u * set + i) * 64u + lane] * f;
+    }
+    if (row >= T) return;
+    const uint32_t qh = kvh * kGroup + (col & 7u), d0 = 32u * set + 4u * grp;
+    if (S == 1u) {
+        uint16_t* d = out + (size_t)row * 2048u + qh * kD + d0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            uint16_t w[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) w[j] = f32_to_bf16(L > 0.f ? o[i][j] / L : 0.f);
+            *reinterpret_cast<uint2*>(d + 16u * i) =
+                make_uint2((uint32_t)w[0] | ((uint32_t)w[1] << 16),
+                           (uint32_t)w[2] | ((uint32_t)w[3] << 16));
+        }
+    } else {
+        float* pw = partials + ((size_t)(row * 16u + qh) * S + s) * kPartial;
+        if (grp == 0u && set == 0u) {
+            pw[0] = M * kScoreScale;
+            pw[1] = L;
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            float* d = pw + 2u + d0 + 16u * i;
+            *reinterpret_cast<float2*>(d) = make_float2(o[i][0], o[i][1]);
+            *reinterpret_cast<float2*>(d + 2) = make_float2(o[i][2], o[i][3]);
+        }
+    }
+}
+
+// Split merge: one wave per (t, qh), lane = dims 2 lane and 2 lane + 1, 4 per
+// workgroup; grid = T * 4. All S records are requested before the first is
+// used (one memory round: 777 rows at base 3001 with 5 splits on the halves
+// 58.6 -> 50.3 us against a 128-thread block per (t, qh) walking the records).
+__global__ void __launch_bounds__(256) prefill_merge_kernel(
+    const float* __restrict__ partials, uint32_t S, uint16_t* __restrict__ out) {
+    const uint32_t bh = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
     const float* base = partials + (size_t)bh * S * kPartial;
+    float2 ml[8], v[8];
+#pragma unroll
+    for (uint32_t i = 0; i < 8u; ++i) {
+        const float* p = base + (size_t)min(i, S - 1u) * kPartial;
+        ml[i] = *reinterpret_cast<const float2*>(p);
+        v[i] = *reinterpret_cast<const float2*>(p + 2u + 2u * lane);
+    }
     float M = -INFINITY;
-    for (uint32_t i = 0; i < S; ++i) {
-        const float* p = base + (size_t)i * kPartial;
-        if (p[1] != 0.f) M = fmaxf(M, p[0]);
+#pragma unroll
+    for (uint32_t i = 0; i < 8u; ++i)
+        if (i < S && ml[i].y != 0.f) M = fmaxf(M, ml[i].x);
+    float L = 0.f, A = 0.f, B = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < 8u; ++i) {
+        if (i >= S || ml[i].y == 0.f) continue;
+        const float f = expf(ml[i].x - M);
+        L += ml[i].y * f;
+        A += v[i].x * f;
+        B += v[i].y * f;
     }
-    float L = 0.f, A = 0.f;
-    for (uint32_t i = 0; i < S; ++i) {
-        const float* p = base + (size_t)i * kPartial;
-        if (p[1] == 0.f) continue;
-        const float f = expf(p[0] - M);
-        L += p[1] * f;
-        A += p[2 + d] * f;
-    }
-    out[(size_t)t * 2048u + (bh & 15u) * kD + d] = f32_to_bf16(L > 0.f ? A / L : 0.f);
+    const uint16_t a = f32_to_bf16(L > 0.f ? A / L : 0.f), b = f32_to_bf16(L > 0.f ? B / L : 0.f);
+    *reinterpret_cast<uint32_t*>(out + (size_t)bh * kD + 2u * lane) =
+        (uint32_t)a | ((uint32_t)b << 16);
 }
 
 }  // namespace
@@ -665,8 +944,8 @@ __global__ void __launch_bounds__(128) prefill_merge_kernel(
 using namespace mckv;
 
 extern "C" mc_status_t mc_kv_debug_prefill_shape(uint32_t shape, uint32_t* previous) {
-    if (shape > mckv::kHalves16 && shape != mckv::kAutoShape) {
-        set_error("mc_kv_debug_prefill_shape: shape %u is not 0, 1, 2 or 0xFFFFFFFF", shape);
+    if (shape > mckv::kSets4 && shape != mckv::kAutoShape) {
+        set_error("mc_kv_debug_prefill_shape: shape %u is not 0..4 or 0xFFFFFFFF", shape);
         return MC_E_INVALID_ARGUMENT;
     }
     const uint32_t prev = mckv::g_shape.exchange(shape);
@@ -738,13 +1017,12 @@ extern "C" mc_status_t mc_kv_debug_prefill_force_timeouts(uint32_t count) {
     return MC_OK;
 }
 
-extern "C" mc_status_t mc_kv_attention_prefill(const uint16_t* d_q_rows, uint32_t tokens,
-                                               const uint32_t* d_base_pos, uint32_t layer,
-                                               const uint32_t* d_page_table,
-                                               const uint16_t* d_kv_pool,
-                                               mc_kv_layout_t layout, uint16_t* d_out,
-                                               float* d_partials, uint32_t S_kv,
-                                               void* stream) {
+namespace mckv {
+mc_status_t prefill_attention(const uint16_t* d_q_rows, uint32_t tokens,
+                              const uint32_t* d_base_pos, uint32_t layer,
+                              const uint32_t* d_page_table, const uint16_t* d_kv_pool,
+                              mc_kv_layout_t layout, uint16_t* d_out, float* d_partials,
+                              uint32_t S_kv, uint32_t keys, void* stream) {
     mckv::TraceRange trace_range("mc_kv_attention_prefill");
     DevLayout ly;
     if (d_q_rows == nullptr || d_base_pos == nullptr || d_page_table == nullptr ||
@@ -757,22 +1035,46 @@ extern "C" mc_status_t mc_kv_attention_prefill(const uint16_t* d_q_rows, uint32_
         return MC_E_INVALID_ARGUMENT;
     }
     hipStream_t st = (hipStream_t)stream;
-    // Shape: 32-row tiles while they give at least two workgroups per CU;
-    // below that 16-row tiles, as two halves on alternate key steps when the
+    // Shape. The key-set workgroups: 4 rows each while that gives every CU at
+    // most one, else 8 (us per layer at base 0: 512 rows 11.0 with 4 rows,
+    // 13.2 with 8; 1024 rows 21.2 / 19.5).
+    // * S_kv = 1: to kSetsRows rows (8 rows against the halves below: 1024
+    //   rows 19.5 / 27.5, at base 8000 109 / 152), and to twice as many where
+    //   the caller knows that the prefix is no longer than the chunk (1500
+    //   rows 25.4 / 35.5, but 107 / 100 at base 4000, where two rounds of
+    //   workgroups pack worse).
+    // * S_kv > 1 is the most key splits: to kSetsSplitRows rows the key sets,
+    //   with no more splits than keep one workgroup per CU (256 rows at base
+    //   2000: 20.9 with 2 splits, 24.6 with 8; 16-row tiles with 8: 23.7).
+    //   Longer chunks keep 16-row tiles and all splits (777 rows at base 3001:
+    //   42.4 with 5 splits, key sets 49.7; at base 0 they would take 16.8
+    //   against 25.0, so a caller that knows its base passes S_kv = 1 there).
+    // Above, 32-row tiles while they give at least two workgroups per CU, and
+    // 16-row tiles below that, as two halves on alternate key steps when the
     // launch has no key splits and at most two 16-row jobs per CU (the
     // heaviest causal tile then sets the time, and the halves take it at
     // twice the rate), else as 4-wave workgroups two per CU. Measured
-    // (base 0): T=2048 67 -> 60 (16 rows) -> 47.5 us (halves), T=4096
-    // 125 -> 118 -> 99.7 us; T=6144 178.5 us with 4-wave workgroups against
+    // (base 0): T=3072 65.2 us with halves against 69.3, T=4096 125 (32 rows)
+    // -> 118 -> 99.7 us; T=6144 178.5 us with 4-wave workgroups against
     // 210 with halves. With S_kv > 1 a tile's split boundaries follow its
-    // last row, so they differ between 32- and 16-row tiles.
+    // last row, so they differ between tile heights.
     const uint32_t ntq32 = (tokens + 31u) / 32u, ntq16 = (tokens + 15u) / 16u;
-    const uint32_t cus = cu_count();
+    const uint32_t jobs8 = kHkv * ((tokens + 7u) / 8u), jobs4 = kHkv * ((tokens + 3u) / 4u);
+    const uint32_t cus = cu_count(), cu = cus ? cus : 256u;
     uint32_t shape = g_shape.load(std::memory_order_relaxed);
     if (shape == kAutoShape) {
-        if (kHkv * ntq32 * S_kv >= kSmallBelow) shape = kRows32;
-        else if (S_kv == 1u && kHkv * ntq16 <= 2u * (cus ? cus : 256u)) shape = kHalves16;
-        else shape = kRows16;
+        const bool short_prefix = keys != 0u && keys / 2u <= tokens;
+        if (tokens <= (S_kv > 1u ? kSetsSplitRows : short_prefix ? 2u * kSetsRows : kSetsRows)) {
+            const uint32_t s4 = std::min(S_kv, cu / jobs4), s8 = std::min(S_kv, cu / jobs8);
+            shape = s4 >= 1u && s4 >= s8 ? kSets4 : kSets8;
+            S_kv = std::max(1u, shape == kSets4 ? s4 : s8);
+        } else if (kHkv * ntq32 * S_kv >= kSmallBelow) {
+            shape = kRows32;
+        } else if (S_kv == 1u && kHkv * ntq16 <= 2u * cu) {
+            shape = kHalves16;
+        } else {
+            shape = kRows16;
+        }
     }
 #define MC_PF_LAUNCH(PG, SM)                                                                 \
     hipLaunchKernelGGL((prefill_attn_kernel<PG, SM>),                                        \
@@ -789,15 +1091,40 @@ extern "C" mc_status_t mc_kv_attention_prefill(const uint16_t* d_q_rows, uint32_
     if (pm == kPageStep) MC_PF_LAUNCH(kPageStep, SM);            \
     else if (pm == kPageHalf) MC_PF_LAUNCH(kPageHalf, SM);       \
     else MC_PF_LAUNCH(kPageRow, SM);
+#define MC_PF_SETS(PG, CG)                                                                        \
+    hipLaunchKernelGGL((prefill_sets_kernel<PG, CG>), dim3((CG == 4 ? jobs8 : jobs4) * S_kv),    \
+                       dim3(64u * CG * kSets), 0, st, d_q_rows, tokens, d_base_pos, layer,       \
+                       d_page_table, d_kv_pool, ly, d_out, d_partials, S_kv)
     switch (shape) {
         case kRows32: MC_PF_PM(kRows32) break;
         case kRows16: MC_PF_PM(kRows16) break;
-        default: MC_PF_PM(kHalves16) break;
+        case kHalves16: MC_PF_PM(kHalves16) break;
+        case kSets8:
+            if (P >= kSetBlock) MC_PF_SETS(true, 4);
+            else MC_PF_SETS(false, 4);
+            break;
+        default:
+            if (P >= kSetBlock) MC_PF_SETS(true, 2);
+            else MC_PF_SETS(false, 2);
+            break;
     }
+#undef MC_PF_SETS
 #undef MC_PF_PM
 #undef MC_PF_LAUNCH
     if (S_kv > 1u)
-        hipLaunchKernelGGL(prefill_merge_kernel, dim3(tokens * 16u), dim3(128), 0, st,
-                           d_partials, S_kv, tokens, d_out);
+        hipLaunchKernelGGL(prefill_merge_kernel, dim3(tokens * 4u), dim3(256), 0, st, d_partials,
+                           S_kv, d_out);
     return check_launch("prefill attention launch failed");
+}
+}  // namespace mckv
+
+extern "C" mc_status_t mc_kv_attention_prefill(const uint16_t* d_q_rows, uint32_t tokens,
+                                               const uint32_t* d_base_pos, uint32_t layer,
+                                               const uint32_t* d_page_table,
+                                               const uint16_t* d_kv_pool,
+                                               mc_kv_layout_t layout, uint16_t* d_out,
+                                               float* d_partials, uint32_t S_kv,
+                                               void* stream) {
+    return mckv::prefill_attention(d_q_rows, tokens, d_base_pos, layer, d_page_table, d_kv_pool,
+                                   layout, d_out, d_partials, S_kv, 0u, stream);
 }

@@ -44,6 +44,7 @@
 
 #include "error.h"
 #include "kv_common.h"
+#include "kv_internal.h"
 #include "mc_kv.h"
 #include "model_internal.h"
 #include "prefill_gemm_table.h"
@@ -432,16 +433,17 @@ void forward_carve(Forward& f, char* p, uint32_t rows, uint32_t logit_rows) {
     f.rows = rows;
 }
 
-// Key splits of a prefill chunk's attention: the reference's count for n
-// rows (kernels.h:517-521: 4096 / n, 1..8), capped so that each split gets
-// at least kSplitKeysMin keys of the chunk's last row. A split of a few
-// 64-key steps gains nothing and costs the merge kernel (a 32-token prompt:
-// 8 splits of 4 keys, attention 8.7 us + merge 5.0 us per layer). Splits
-// change the result's rounding only.
+// Key splits of a prefill chunk's attention: none where the prefix is at most
+// twice the chunk (the unsplit key-set shapes are then the faster ones: 1024
+// rows 19.5 us against 31.0 with 2 splits; 640 rows after 1280 about equal),
+// else the reference's count for n rows (kernels.h:517-521: 4096 / n, 1..8),
+// capped so that each split gets at least kSplitKeysMin keys of the chunk's
+// last row. Splits change the result's rounding only.
 constexpr uint32_t kSplitKeysMin = 512u;
 uint32_t prefill_splits(uint32_t n, uint32_t keys) {
     const uint32_t s = mc_kv_prefill_split_kv(n);
     if (keys == 0u) return s;
+    if (keys / 3u <= n) return 1u;
     const uint32_t cap = keys / kSplitKeysMin;
     return s < cap ? s : (cap < 1u ? 1u : cap);
 }
@@ -491,8 +493,8 @@ mc_status_t forward_prefill_rows(const Forward& f, const int32_t* d_ids, uint32_
         if (pending != nullptr) std::swap(cur, other);
         FWD_OR_RETURN(mc_kv_rope_append(f.qkv, n, f.d_seq_len, l, f.d_pt, f.pool, f.layout, kTheta,
                                         rope_table_off() ? nullptr : f.inv_freq, st));
-        FWD_OR_RETURN(mc_kv_attention_prefill(f.qkv, n, f.d_seq_len, l, f.d_pt, f.pool, f.layout,
-                                              f.attn, S > 1u ? f.pf_partials : nullptr, S, st));
+        FWD_OR_RETURN(prefill_attention(f.qkv, n, f.d_seq_len, l, f.d_pt, f.pool, f.layout, f.attn,
+                                        S > 1u ? f.pf_partials : nullptr, S, f.keys, st));
         FWD_OR_RETURN(mc_model_gemv(w.o[l], f.attn, kHidden, f.o_out, kHidden, n, kHidden,
                                     kHidden, st));
         FWD_OR_RETURN(mc_model_gemv_resnorm_swiglu(w.gate_up[l], cur, f.o_out, w.norm2[l], other,
@@ -567,8 +569,8 @@ mc_status_t forward_prefill(const Forward& f, const int32_t* d_ids, uint32_t n, 
         FWD_OR_RETURN(proj(f.normed, w.qkv[l], kQkvCols, kHidden, f.qkv));
         FWD_OR_RETURN(mc_kv_rope_append(f.qkv, n, f.d_seq_len, l, f.d_pt, f.pool, f.layout, kTheta,
                                         rope_table_off() ? nullptr : f.inv_freq, st));
-        FWD_OR_RETURN(mc_kv_attention_prefill(f.qkv, n, f.d_seq_len, l, f.d_pt, f.pool, f.layout,
-                                              f.attn, S > 1u ? f.pf_partials : nullptr, S, st));
+        FWD_OR_RETURN(prefill_attention(f.qkv, n, f.d_seq_len, l, f.d_pt, f.pool, f.layout, f.attn,
+                                        S > 1u ? f.pf_partials : nullptr, S, f.keys, st));
         FWD_OR_RETURN(proj(f.attn, w.o[l], kHidden, kHidden, f.o_out));
         FWD_OR_RETURN(
             mc_model_rmsnorm_rows(res, f.o_out, w.norm2[l], f.normed, n, kHidden, kRmsEps, st));

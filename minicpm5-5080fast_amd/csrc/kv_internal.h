@@ -26,4 +26,14 @@ mc_status_t launch_synth_qkv_batch(uint16_t* rows, uint32_t n,
 // count; MC_E_INTERNAL (with a message) when it is non-zero.
 mc_status_t prefill_barrier_check(const char* who);
 
+
+// mc_kv_attention_prefill for a caller that knows on the host how many keys
+// the chunk's last row attends (keys; 0 = not known), which decides the
+// workgroup shape of some row counts.
+mc_status_t prefill_attention(const uint16_t* d_q_rows, uint32_t tokens,
+                              const uint32_t* d_base_pos, uint32_t layer,
+                              const uint32_t* d_page_table, const uint16_t* d_kv_pool,
+                              mc_kv_layout_t layout, uint16_t* d_out, float* d_partials,
+                              uint32_t S_kv, uint32_t keys, void* stream);
+
 }  // namespace mckv
