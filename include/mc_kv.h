@@ -135,6 +135,12 @@ mc_status_t mc_kv_rope_append(uint16_t* d_qkv, uint32_t tokens,
                               mc_kv_layout_t layout, double rope_theta,
                               const float* d_inv_freq, void* stream);
 
+/* cos / sin of the 64 rotate pairs of positions *d_base_pos + t, as 64 float
+ * pairs from column 2048 of each token's qkv row (for
+ * mc_model_gemm_tiles_rope). rope_theta / d_inv_freq as above. */
+mc_status_t mc_kv_rope_table(uint16_t* d_qkv, uint32_t tokens, const uint32_t* d_base_pos,
+                             double rope_theta, const float* d_inv_freq, void* stream);
+
 /* ---- decode attention (split-KV flash decoding) ---- */
 
 /* launch_attention_decode (kernels.h:369-388, attention_decode.cu:1840-1964).

@@ -19,6 +19,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "mc_kv.h"
 #include "minicpm_runtime.h"
 
 #ifdef __cplusplus
@@ -106,6 +107,42 @@ mc_status_t mc_model_gemv_swiglu(const uint16_t* d_w, const uint16_t* d_gate_up,
 mc_status_t mc_model_gemm_rows(const uint16_t* d_w, const uint16_t* d_x, uint32_t ldx,
                                uint16_t* d_y, uint32_t ldy, uint32_t M, uint32_t N, uint32_t K,
                                uint32_t swiglu, void* stream);
+
+/* Tile GEMM of a prefill chunk: d_y[m][n] = bf16(sum_k d_w[n][k] *
+ * d_x[m][k]) with fp32 accumulation, or, with swiglu = 1 (d_w [2N][K]: gate
+ * rows, then up rows), d_y[m][n] = bf16(silu(g) * u) of the rows n and N + n
+ * rounded to bf16, as mc_model_gemm_rows. With d_partials instead of d_y the
+ * fp32 sums of each of `splits` equal K ranges go to d_partials[split][M][N]
+ * (splits > 1 needs it; not with swiglu). Rows are contiguous (strides K and
+ * N), N a multiple of 64, K of 128 * splits, pointers 16-byte aligned. shape: MC_MODEL_GEMM_TILES_AUTO (least estimated
+ * time) or a row 0..MC_MODEL_GEMM_TILES_SHAPES - 1 of the tile table
+ * (MC_E_INVALID_ARGUMENT where it does not take the sizes). No reference
+ * counterpart: the reference runs multi-token chunks through cuBLAS
+ * (forward.cpp:200-420). */
+#define MC_MODEL_GEMM_TILES_SHAPES 18u
+#define MC_MODEL_GEMM_TILES_AUTO 0xFFFFFFFFu
+mc_status_t mc_model_gemm_tiles(const uint16_t* d_w, const uint16_t* d_x, uint16_t* d_y,
+                                float* d_partials, uint32_t M, uint32_t N, uint32_t K,
+                                uint32_t swiglu, uint32_t splits, uint32_t shape, void* stream);
+
+/* The qkv projection of a prefill chunk with RoPE and the K/V append as its
+ * epilogue, on the same tiles: rows d_x [M][K], weights d_w [2560][K]; the
+ * rotated q heads go to d_qkv [M][2560], rotated k and v to the pages of
+ * positions *d_base_pos + m (as mc_kv_rope_append of the rounded projection,
+ * bit for bit). The k / v columns of d_qkv are not written: on entry they hold
+ * the rows' cos / sin pairs (mc_kv_rope_table). K as above. */
+mc_status_t mc_model_gemm_tiles_rope(const uint16_t* d_w, const uint16_t* d_x, uint16_t* d_qkv,
+                                     uint32_t M, uint32_t K, const uint32_t* d_base_pos,
+                                     uint32_t layer, const uint32_t* d_page_table,
+                                     uint16_t* d_kv_pool, mc_kv_layout_t layout, uint32_t shape,
+                                     void* stream);
+
+/* mc_model_rmsnorm_rows over rows of 2048 whose addend is the sum of `splits`
+ * (1..8) fp32 partials d_partials[split][rows][2048] (16-byte aligned), added
+ * in split order and rounded to bf16 first. */
+mc_status_t mc_model_rmsnorm_splits(uint16_t* d_res, const float* d_partials, uint32_t splits,
+                                    const uint16_t* d_weight, uint16_t* d_out, uint32_t rows,
+                                    float eps, void* stream);
 
 /* ---- FP8 projections (precision MC_FP8: single-token forwards) ----
  * d_w: e4m3 codes [N][K] (uint8, 16-byte aligned rows), d_scale: fp32 [N]

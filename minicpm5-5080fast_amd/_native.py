@@ -57,6 +57,7 @@ _SIGS = {
     "mc_kv_pool_session_pages": (_u32, [_P, _u32]),
     "mc_kv_pool_session_table": (_u32, [_P, _u32, _P, _u32]),
     "mc_kv_rope_inv_freq_init": (C.c_int, [_P, C.c_double, _P]),
+    "mc_kv_rope_table": (C.c_int, [_P, _u32, _P, C.c_double, _P, _P]),
     "mc_kv_rope_append": (C.c_int, [_P, _u32, _P, _u32, _P, _P, LayoutT, C.c_double,
                                     _P, _P]),
     "mc_kv_attention_decode": (C.c_int, [_P, _P, _u32, _P, _P, LayoutT, _P, _u32, _P,
@@ -86,6 +87,10 @@ _SIGS = {
     "mc_model_rmsnorm_rows": (C.c_int, [_P, _P, _P, _P, _u32, _u32, C.c_float, _P]),
     "mc_model_swiglu_rows": (C.c_int, [_P, _P, _u32, _u32, _P]),
     "mc_model_gemv": (C.c_int, [_P, _P, _u32, _P, _u32, _u32, _u32, _u32, _P]),
+    "mc_model_gemm_tiles": (C.c_int, [_P, _P, _P, _P, _u32, _u32, _u32, _u32, _u32, _u32, _P]),
+    "mc_model_gemm_tiles_rope": (C.c_int, [_P, _P, _P, _u32, _u32, _P, _u32, _P, _P, LayoutT,
+                                           _u32, _P]),
+    "mc_model_rmsnorm_splits": (C.c_int, [_P, _P, _u32, _P, _P, _u32, C.c_float, _P]),
     "mc_model_gemm_rows": (C.c_int, [_P, _P, _u32, _P, _u32, _u32, _u32, _u32, _u32, _P]),
     "mc_model_gemv_resnorm": (C.c_int, [_P, _P, _P, _P, _P, _u32, _P, _u32, _u32, _u32,
                                         C.c_float, _P]),

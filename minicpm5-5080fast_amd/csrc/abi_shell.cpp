@@ -219,7 +219,7 @@ struct SessionImpl {
     Breakdown bd;
     // with weights
     Forward fwd;
-    void* blas = nullptr;  // prefill GEMM libraries (prefill_blas_create)
+    void* blas = nullptr;  // prefill GEMM library (prefill_blas_create)
     int32_t* h_emit = nullptr;  // pinned: the token a decode returns
 };
 
@@ -547,8 +547,9 @@ mc_status_t mc_session_create(mc_model_t model, mc_session_t* out_session) {
     s->max_chunks = mc_kv_decode_max_chunks(m->max_ctx, s->chunk_pos);
     s->act_rows = std::min(m->max_ctx, prefill_chunk_tokens());
     const size_t pool_b = (size_t)mc_kv_total_elems(s->layout) * 2u;
-    // With weights: the prefill projections' rocBLAS and hipBLASLt handles get
-    // their device workspace from the arena, so neither allocates after create.
+    // With weights: the rocBLAS handle of the prefill projections (used when an
+    // environment variable asks for it) gets its device workspace from the
+    // arena, so it does not allocate after create.
     size_t blas_ws = 0;
     if (m->weights) {
         const mc_status_t bs = prefill_blas_create(&s->blas, &blas_ws);

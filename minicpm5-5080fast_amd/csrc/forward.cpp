@@ -12,9 +12,12 @@
 //   and logits are bf16.
 //
 // MI355X mapping:
-//   * prefill (T rows): projections through rocBLAS GEMM (bf16 in/out, fp32
-//     compute), RMSNorm / residual-add kernels, SwiGLU, the paged prefill
-//     attention; the lm_head of the last row through the GEMV;
+//   * prefill (T rows): projections through the row GEMM (9..32 rows), the
+//     tile GEMM (gemm_tiles.hip; the SwiGLU as gate_up's epilogue, K splits of
+//     o and down summed by the norm that follows); RMSNorm / residual-add
+//     kernels, the paged prefill attention; the lm_head of the last row
+//     through the GEMV. rocBLAS runs them only when an environment variable
+//     asks for it (MC_PREFILL_GEMM_DEFAULT, MC_PREFILL_ROWS_GEMV_OFF);
 //   * decode (one row) and batch steps (n <= 8 rows): every projection is the
 //     HBM-streaming GEMV of model_kernels.hip, with the residual add + RMSNorm
 //     fused into the GEMV that consumes it (qkv, gate_up, lm_head) and the
@@ -26,7 +29,6 @@
 //     workgroups still reading the old one. Attention is the phase0 decode
 //     (RoPE + K/V append + split-KV attention in one chunk kernel).
 #include <hip/hip_runtime.h>
-#include <hipblaslt/hipblaslt.h>
 #include <rocblas/rocblas.h>
 
 #include <algorithm>
@@ -35,19 +37,17 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <mutex>
 #include <new>
 #include <string>
-#include <unordered_map>
 #include <utility>
 #include <vector>
 
 #include "error.h"
+#include "gemm_tiles.h"
 #include "kv_common.h"
 #include "kv_internal.h"
 #include "mc_kv.h"
 #include "model_internal.h"
-#include "prefill_gemm_table.h"
 #include "trace.h"
 
 namespace mckv {
@@ -73,171 +73,68 @@ size_t a256(size_t x) { return (x + 255u) & ~size_t(255); }
         if (_s != MC_OK) return _s;     \
     } while (0)
 
-// The tuned table of the rocBLAS this process resolved (by its version
-// string), or null.
+// MC_PREFILL_GEMM_DEFAULT=1 (read once per process): every projection of
+// chunks that are not run row by row goes through rocBLAS.
 bool gemm_defaults_only() {
     static const bool on = std::getenv("MC_PREFILL_GEMM_DEFAULT") != nullptr;
     return on;
 }
 
-const PrefillGemmTable* gemm_table() {
-    static const PrefillGemmTable* t = []() -> const PrefillGemmTable* {
-        if (gemm_defaults_only()) return nullptr;
-        char ver[256] = {0};
-        if (rocblas_get_version_string(ver, sizeof(ver)) != rocblas_status_success)
-            return nullptr;
-        for (const PrefillGemmTable& e : kPrefillGemmTables)
-            if (std::strcmp(e.rocblas_version, ver) == 0) return &e;
-        return nullptr;
-    }();
-    return t;
-}
-
-static_assert(sizeof(kPrefillGemmRocm) / sizeof(kPrefillGemmRocm[0]) <= 64u &&
-                  sizeof(kPrefillGemmTorch) / sizeof(kPrefillGemmTorch[0]) <= 64u,
-              "a table row is one bit of gemm_bf16's rejection mask");
-
-// Row of the tuned table for an M x N x K projection: the largest tuned M not
-// above M; -1 below the smallest, for other shapes or without a table.
-int gemm_row(const PrefillGemmTable* t, uint32_t M, uint32_t N, uint32_t K) {
-    int row = -1;
-    if (t == nullptr) return row;
-    for (uint32_t i = 0; i < t->count; ++i) {
-        const PrefillGemmSolution& e = t->rows[i];
-        if (e.n == N && e.k == K && e.m <= M) row = (int)i;
-    }
-    return row;
-}
-
-// The prefill projections' GEMM libraries of one session.
+// The prefill projections' GEMM library of one session.
 struct PrefillBlas {
     rocblas_handle rb = nullptr;
-    hipblasLtHandle_t lt = nullptr;
-    hipblasLtMatmulDesc_t desc = nullptr;  // y^T = W^T(op T) . x^T, fp32 compute
-    void* ws = nullptr;
-    size_t ws_bytes = 0;
 };
 
-// hipBLASLt rows: chunks of kLtMinRows..kLtMaxRows rows without a tuned
-// rocBLAS solution go through hipBLASLt with the heuristic's first algorithm,
-// looked up once per (M, N, K) per process. Through PyTorch's libraries a
-// rocblas_gemm_ex call takes ~16 us of host time whatever the size, a
-// hipblasLtMatmul call ~9 us, with kernels of the same speed; measured, the
-// prefill of 17..256 tokens is 3-11% faster this way. Larger chunks stay on
-// rocBLAS (its tuned table; the host time is hidden behind the kernels).
-constexpr uint32_t kLtMinRows = 17u, kLtMaxRows = 1023u;
-
-struct LtAlgoCache {
-    std::mutex mu;
-    std::unordered_map<uint64_t, hipblasLtMatmulAlgo_t> algos;
-    std::unordered_map<uint64_t, bool> failed;
-};
-LtAlgoCache& lt_cache() {
-    static LtAlgoCache c;
-    return c;
-}
-
-// y[M][N] = x[M][K] . W[N][K]^T through hipBLASLt; false (nothing launched)
-// when hipBLASLt has no algorithm for the shape or rejects the call.
-bool gemm_lt(const PrefillBlas& b, hipStream_t st, const uint16_t* x, uint32_t M,
-             const uint16_t* W, uint32_t N, uint32_t K, uint16_t* y) {
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    const uint64_t key = ((uint64_t)(uint32_t)dev << 56) ^ ((uint64_t)M << 32) ^
-                         ((uint64_t)N << 16) ^ (uint64_t)K;
-    hipblasLtMatrixLayout_t la = nullptr, lb = nullptr, lc = nullptr;
-    bool ok = hipblasLtMatrixLayoutCreate(&la, HIP_R_16BF, K, N, K) == HIPBLAS_STATUS_SUCCESS &&
-              hipblasLtMatrixLayoutCreate(&lb, HIP_R_16BF, K, M, K) == HIPBLAS_STATUS_SUCCESS &&
-              hipblasLtMatrixLayoutCreate(&lc, HIP_R_16BF, N, M, N) == HIPBLAS_STATUS_SUCCESS;
-    hipblasLtMatmulAlgo_t algo{};
-    if (ok) {
-        LtAlgoCache& c = lt_cache();
-        std::lock_guard<std::mutex> lk(c.mu);
-        auto it = c.algos.find(key);
-        if (it != c.algos.end()) {
-            algo = it->second;
-        } else if (c.failed.count(key)) {
-            ok = false;
-        } else {
-            hipblasLtMatmulPreference_t pref = nullptr;
-            hipblasLtMatmulHeuristicResult_t res{};
-            int n = 0;
-            uint64_t wsz = b.ws_bytes;
-            ok = hipblasLtMatmulPreferenceCreate(&pref) == HIPBLAS_STATUS_SUCCESS &&
-                 hipblasLtMatmulPreferenceSetAttribute(
-                     pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &wsz, sizeof(wsz)) ==
-                     HIPBLAS_STATUS_SUCCESS &&
-                 hipblasLtMatmulAlgoGetHeuristic(b.lt, b.desc, la, lb, lc, lc, pref, 1, &res,
-                                                 &n) == HIPBLAS_STATUS_SUCCESS &&
-                 n > 0 && res.state == HIPBLAS_STATUS_SUCCESS && res.workspaceSize <= b.ws_bytes;
-            if (pref) (void)hipblasLtMatmulPreferenceDestroy(pref);
-            if (ok) {
-                algo = res.algo;
-                c.algos.emplace(key, algo);
-            } else {
-                c.failed.emplace(key, true);
-            }
-        }
-    }
-    if (ok) {
-        const float alpha = 1.f, beta = 0.f;
-        ok = hipblasLtMatmul(b.lt, b.desc, &alpha, W, la, x, lb, &beta, y, lc, y, lc, &algo, b.ws,
-                             b.ws_bytes, st) == HIPBLAS_STATUS_SUCCESS;
-    }
-    if (la) (void)hipblasLtMatrixLayoutDestroy(la);
-    if (lb) (void)hipblasLtMatrixLayoutDestroy(lb);
-    if (lc) (void)hipblasLtMatrixLayoutDestroy(lc);
-    return ok;
-}
-
-// y[M][N] = x[M][K] . W[N][K]^T (column-major view: C(N x M) = W^T(N x K) .
-// x^T(K x M)). A shape with a tuned rocBLAS solution runs it; an index that
-// rocBLAS rejects (it checks one against the problem before launching) reruns
-// the call on the default heuristic and leaves that table row on it for the
-// rest of the process. Other shapes of kLtMinRows..kLtMaxRows rows go through
-// hipBLASLt, the rest (and whatever hipBLASLt declines) through rocBLAS's
-// default heuristic. MC_PREFILL_GEMM_DEFAULT=1 sends every projection to
-// rocBLAS's default heuristic (the measured A/B of the tables and the
-// hipBLASLt rows).
+// y[M][N] = x[M][K] . W[N][K]^T on rocBLAS (column-major view: C(N x M) =
+// W^T(N x K) . x^T(K x M)).
 mc_status_t gemm_bf16(const Forward& f, const uint16_t* x, uint32_t M, const uint16_t* W,
                       uint32_t N, uint32_t K, uint16_t* y) {
-    const PrefillBlas& b = *static_cast<const PrefillBlas*>(f.blas);
-    const PrefillGemmTable* t = gemm_table();
-    const int row = gemm_row(t, M, N, K);
-    // rows whose index this process's rocBLAS rejected
-    static std::atomic<uint64_t> rejected{0};
-    const uint64_t bit = row >= 0 ? uint64_t(1) << row : 0u;
-    const int32_t idx = row >= 0 && !(rejected.load(std::memory_order_relaxed) & bit)
-                            ? t->rows[row].index
-                            : 0;
-    if (idx == 0 && M >= kLtMinRows && M <= kLtMaxRows && !gemm_defaults_only() &&
-        gemm_lt(b, f.st, x, M, W, N, K, y))
-        return MC_OK;
-    rocblas_handle h = b.rb;
+    rocblas_handle h = static_cast<const PrefillBlas*>(f.blas)->rb;
     if (rocblas_set_stream(h, f.st) != rocblas_status_success) {
         set_error("prefill GEMM: rocblas_set_stream failed");
         return MC_E_CUDA;
     }
     const float alpha = 1.f, beta = 0.f;
-    auto run = [&](int32_t i) {
-        return rocblas_gemm_ex(
-            h, rocblas_operation_transpose, rocblas_operation_none, (rocblas_int)N,
-            (rocblas_int)M, (rocblas_int)K, &alpha, W, rocblas_datatype_bf16_r, (rocblas_int)K, x,
-            rocblas_datatype_bf16_r, (rocblas_int)K, &beta, y, rocblas_datatype_bf16_r,
-            (rocblas_int)N, y, rocblas_datatype_bf16_r, (rocblas_int)N, rocblas_datatype_f32_r,
-            i ? rocblas_gemm_algo_solution_index : rocblas_gemm_algo_standard, i, 0);
-    };
-    rocblas_status s = run(idx);
-    if (s != rocblas_status_success && idx != 0) {
-        rejected.fetch_or(bit, std::memory_order_relaxed);
-        s = run(0);
-    }
+    const rocblas_status s = rocblas_gemm_ex(
+        h, rocblas_operation_transpose, rocblas_operation_none, (rocblas_int)N, (rocblas_int)M,
+        (rocblas_int)K, &alpha, W, rocblas_datatype_bf16_r, (rocblas_int)K, x,
+        rocblas_datatype_bf16_r, (rocblas_int)K, &beta, y, rocblas_datatype_bf16_r,
+        (rocblas_int)N, y, rocblas_datatype_bf16_r, (rocblas_int)N, rocblas_datatype_f32_r,
+        rocblas_gemm_algo_standard, 0, 0);
     if (s != rocblas_status_success) {
         set_error("prefill GEMM (%u x %u x %u): rocblas_gemm_ex failed: %s", M, N, K,
                   rocblas_status_to_string(s));
         return MC_E_CUDA;
     }
     return MC_OK;
+}
+
+// How a chunk of n rows runs its projections: a tile shape and K splits each,
+// or splits = 0 for rocBLAS (MC_PREFILL_GEMM_DEFAULT=1 sends all there).
+struct PrefillPlan {
+    GemmPlan qkv, o, gate_up, down;
+    bool rope = false;  // qkv's tiles rotate and append (no RoPE kernel)
+};
+PrefillPlan prefill_plan(const Forward& f, uint32_t n) {
+    PrefillPlan p;
+    if (gemm_defaults_only() || n <= MC_MODEL_GEMM_ROWS_MAX) return p;
+    p.gate_up = gemm_tiles_plan(n, kInter, kHidden, TileEnd::kSwiglu, 1u, 1u);
+    // The rope form saves the RoPE kernel (3.5 us and 2.4 ns per row with its
+    // launch gap) but not every shape takes it.
+    float plain_us, rope_us;
+    p.qkv = gemm_tiles_plan(n, kQkvCols, kHidden, TileEnd::kPlain, 1u, 1u, &plain_us);
+    const GemmPlan r = gemm_tiles_plan(n, kQkvCols, kHidden, TileEnd::kRope, 1u, 1u, &rope_us);
+    if (rope_us < plain_us + 3.5f + 0.0024f * (float)n) {
+        p.qkv = r;
+        p.rope = true;
+    }
+    // the split sums [splits][n][kHidden] fp32 lie in the gate_up buffer of
+    // f.rows rows of 2 kInter bf16
+    const uint32_t fit = (uint32_t)((size_t)f.rows * 2u * kInter * 2u / ((size_t)n * kHidden * 4u));
+    const uint32_t most = fit < 8u ? fit : 8u;
+    p.o = gemm_tiles_plan(n, kHidden, kHidden, TileEnd::kPlain, 1u, most);
+    p.down = gemm_tiles_plan(n, kHidden, kInter, TileEnd::kPlain, 1u, most);
+    return p;
 }
 
 // Device workspace handed to the prefill projections' rocBLAS handle. With a
@@ -360,18 +257,6 @@ mc_status_t prefill_blas_create(void** out, size_t* ws_bytes) {
         set_error("mc_session_create: rocblas_create_handle failed");
         return MC_E_CUDA;
     }
-    const hipblasOperation_t ta = HIPBLAS_OP_T, tb = HIPBLAS_OP_N;
-    if (hipblasLtCreate(&b->lt) != HIPBLAS_STATUS_SUCCESS ||
-        hipblasLtMatmulDescCreate(&b->desc, HIPBLAS_COMPUTE_32F, HIP_R_32F) !=
-            HIPBLAS_STATUS_SUCCESS ||
-        hipblasLtMatmulDescSetAttribute(b->desc, HIPBLASLT_MATMUL_DESC_TRANSA, &ta, sizeof(ta)) !=
-            HIPBLAS_STATUS_SUCCESS ||
-        hipblasLtMatmulDescSetAttribute(b->desc, HIPBLASLT_MATMUL_DESC_TRANSB, &tb, sizeof(tb)) !=
-            HIPBLAS_STATUS_SUCCESS) {
-        prefill_blas_destroy(b);
-        set_error("mc_session_create: hipBLASLt handle or matmul descriptor creation failed");
-        return MC_E_CUDA;
-    }
     *out = b;
     return MC_OK;
 }
@@ -384,16 +269,12 @@ mc_status_t prefill_blas_workspace(void* hv, void* ws, size_t ws_bytes) {
                   rocblas_status_to_string(st));
         return MC_E_CUDA;
     }
-    b->ws = ws;  // hipBLASLt takes it per call
-    b->ws_bytes = ws_bytes;
     return MC_OK;
 }
 
 void prefill_blas_destroy(void* hv) {
     PrefillBlas* b = static_cast<PrefillBlas*>(hv);
     if (b == nullptr) return;
-    if (b->desc) (void)hipblasLtMatmulDescDestroy(b->desc);
-    if (b->lt) (void)hipblasLtDestroy(b->lt);
     if (b->rb) (void)rocblas_destroy_handle(b->rb);
     delete b;
 }
@@ -451,10 +332,8 @@ uint32_t prefill_splits(uint32_t n, uint32_t keys) {
 // Projections of short prefill chunks (whole model, 42 layers, best of 5;
 // library GEMMs in parentheses): 2..8 tokens through forward_prefill_rows
 // 1.74-2.16 ms (3.60-3.67), 9..32 tokens through the row GEMM 2.45-3.31 ms
-// (3.30-3.74); at 33-64 tokens the row GEMM measured slower than hipBLASLt
-// (its activation reads grow with the rows on each of the N / 16
-// workgroups). MC_PREFILL_ROWS_GEMV_OFF=1 sends chunks of 2..32 tokens
-// through the GEMM libraries as well (the measured A/B).
+// (3.30-3.74). MC_PREFILL_ROWS_GEMV_OFF=1 sends chunks of 2..32 tokens
+// through rocBLAS as well (the measured A/B).
 bool prefill_rows_gemv_off() {
     static const bool off = std::getenv("MC_PREFILL_ROWS_GEMV_OFF") != nullptr;
     return off;
@@ -555,38 +434,70 @@ mc_status_t forward_prefill(const Forward& f, const int32_t* d_ids, uint32_t n, 
     FWD_OR_RETURN(mc_model_embedding_gather(w.embedding, d_ids, nullptr, res, kHidden, n, st));
     FWD_OR_RETURN(mc_model_rmsnorm_rows(res, nullptr, w.norm1[0], f.normed, n, kHidden, kRmsEps, st));
     const uint32_t S = prefill_splits(n, f.keys);
-    // 9..32 rows: the projections through the row GEMM (the gate_up one with
-    // the SwiGLU as its epilogue), larger chunks through the GEMM libraries
+    // 9..32 rows: the projections through the row GEMM; larger chunks: the
+    // tile GEMM
     const bool rows = n >= MC_MODEL_GEMM_ROWS_MIN && n <= MC_MODEL_GEMM_ROWS_MAX &&
                       !prefill_rows_gemv_off();
-    auto proj = [&](const uint16_t* x, const uint16_t* W, uint32_t N, uint32_t K, uint16_t* y) {
-        return rows ? mc_model_gemm_rows(W, x, K, y, N, n, N, K, 0u, st)
-                    : gemm_bf16(f, x, n, W, N, K, y);
+    const PrefillPlan plan = prefill_plan(f, n);
+    const float* inv_freq = rope_table_off() ? nullptr : f.inv_freq;
+    DevLayout ly;
+    if (!layout_valid(f.layout, &ly)) {
+        set_error("forward_prefill: invalid KV layout");
+        return MC_E_INTERNAL;
+    }
+    if (plan.rope) FWD_OR_RETURN(mc_kv_rope_table(f.qkv, n, f.d_seq_len, kTheta, inv_freq, st));
+    auto proj = [&](const uint16_t* x, const uint16_t* W, uint32_t N, uint32_t K, uint16_t* y,
+                    const GemmPlan& p) {
+        if (rows) return mc_model_gemm_rows(W, x, K, y, N, n, N, K, 0u, st);
+        if (p.splits == 0u) return gemm_bf16(f, x, n, W, N, K, y);
+        return gemm_tiles({x, W, y, nullptr, n, N, K, false}, p, st);
+    };
+    // residual += x . W^T (kHidden columns), then the next norm; with K splits
+    // the fp32 sums pass through the gate_up buffer (unused by the tile path)
+    auto proj_norm = [&](const uint16_t* x, const uint16_t* W, uint32_t K, uint16_t* y,
+                         const GemmPlan& p, const uint16_t* norm) {
+        if (rows || p.splits <= 1u) {
+            const mc_status_t r = proj(x, W, kHidden, K, y, p);
+            return r != MC_OK ? r
+                              : mc_model_rmsnorm_rows(res, y, norm, f.normed, n, kHidden, kRmsEps,
+                                                      st);
+        }
+        float* part = reinterpret_cast<float*>(f.gate_up);
+        const mc_status_t r = gemm_tiles({x, W, nullptr, part, n, kHidden, K, false}, p, st);
+        return r != MC_OK ? r
+                          : mc_model_rmsnorm_splits(res, part, p.splits, norm, f.normed, n,
+                                                    kRmsEps, st);
     };
     for (uint32_t l = 0; l < kModelLayers; ++l) {
         if (layer_dump)
             FWD_OR_RETURN(dump_bf16(dump_name("layer", l, "hidden_in.f32"), res_last, kHidden, st));
-        FWD_OR_RETURN(proj(f.normed, w.qkv[l], kQkvCols, kHidden, f.qkv));
-        FWD_OR_RETURN(mc_kv_rope_append(f.qkv, n, f.d_seq_len, l, f.d_pt, f.pool, f.layout, kTheta,
-                                        rope_table_off() ? nullptr : f.inv_freq, st));
+        if (plan.rope) {
+            FWD_OR_RETURN(gemm_tiles({f.normed, w.qkv[l], f.qkv, nullptr, n, kQkvCols, kHidden,
+                                      false, {f.d_seq_len, f.d_pt, f.pool, ly, l, 0u}},
+                                     plan.qkv, st));
+        } else {
+            FWD_OR_RETURN(proj(f.normed, w.qkv[l], kQkvCols, kHidden, f.qkv, plan.qkv));
+            FWD_OR_RETURN(mc_kv_rope_append(f.qkv, n, f.d_seq_len, l, f.d_pt, f.pool, f.layout,
+                                            kTheta, inv_freq, st));
+        }
         FWD_OR_RETURN(prefill_attention(f.qkv, n, f.d_seq_len, l, f.d_pt, f.pool, f.layout, f.attn,
                                         S > 1u ? f.pf_partials : nullptr, S, f.keys, st));
-        FWD_OR_RETURN(proj(f.attn, w.o[l], kHidden, kHidden, f.o_out));
-        FWD_OR_RETURN(
-            mc_model_rmsnorm_rows(res, f.o_out, w.norm2[l], f.normed, n, kHidden, kRmsEps, st));
+        FWD_OR_RETURN(proj_norm(f.attn, w.o[l], kHidden, f.o_out, plan.o, w.norm2[l]));
         if (layer_dump)
             FWD_OR_RETURN(dump_bf16(dump_name("layer", l, "attn_out.f32"), res_last, kHidden, st));
         if (rows) {
             FWD_OR_RETURN(mc_model_gemm_rows(w.gate_up[l], f.normed, kHidden, f.mlp, kInter, n,
                                              kInter, kHidden, 1u, st));
+        } else if (plan.gate_up.splits != 0u) {
+            FWD_OR_RETURN(gemm_tiles({f.normed, w.gate_up[l], f.mlp, nullptr, n, kInter, kHidden,
+                                      true},
+                                     plan.gate_up, st));
         } else {
             FWD_OR_RETURN(gemm_bf16(f, f.normed, n, w.gate_up[l], 2u * kInter, kHidden, f.gate_up));
             FWD_OR_RETURN(mc_model_swiglu_rows(f.gate_up, f.mlp, n, kInter, st));
         }
-        FWD_OR_RETURN(proj(f.mlp, w.down[l], kHidden, kInter, f.down));
-        const uint16_t* next_norm = l + 1u < kModelLayers ? w.norm1[l + 1u] : w.final_norm;
-        FWD_OR_RETURN(
-            mc_model_rmsnorm_rows(res, f.down, next_norm, f.normed, n, kHidden, kRmsEps, st));
+        FWD_OR_RETURN(proj_norm(f.mlp, w.down[l], kInter, f.down, plan.down,
+                                l + 1u < kModelLayers ? w.norm1[l + 1u] : w.final_norm));
         if (layer_dump)
             FWD_OR_RETURN(dump_bf16(dump_name("layer", l, "mlp_out.f32"), res_last, kHidden, st));
     }

@@ -29,6 +29,7 @@
 // pairing order (lane_reduce_scatter).
 #include <hip/hip_runtime.h>
 
+#include "bf16_math.h"
 #include "error.h"
 #include "kv_common.h"
 #include "mc_model.h"
@@ -37,7 +38,6 @@
 namespace mckv {
 namespace {
 
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kThreads = 256;
@@ -58,14 +58,6 @@ __device__ __forceinline__ uint4 ld_stream(const uint16_t* p) {
 }
 __device__ __forceinline__ uint4 ld16(const uint16_t* p) {
     return *reinterpret_cast<const uint4*>(p);
-}
-__device__ __forceinline__ float lo_f(uint32_t u) { return __uint_as_float(u << 16); }
-__device__ __forceinline__ float hi_f(uint32_t u) { return __uint_as_float(u & 0xFFFF0000u); }
-// Two fp32 -> bf16 round-to-nearest-even conversions in one v_cvt_pk_bf16_f32
-// (a in the low half).
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){a, b}, bf16x2_t));
 }
 
 // Sum over the 64 lanes, every lane receiving the total: xor 1 and xor 2
@@ -167,6 +159,28 @@ __global__ void __launch_bounds__(kThreads)
 // ---- RMSNorm rows, optionally after the residual add ----
 // grid = rows, block = 256. Each thread owns the same 8-element chunks in
 // both passes, so re-reading its own residual stores needs no barrier.
+__device__ __forceinline__ uint4 add8(const uint4& v, const uint4& a) {
+    return make_uint4(pack2(lo_f(v.x) + lo_f(a.x), hi_f(v.x) + hi_f(a.x)),
+                      pack2(lo_f(v.y) + lo_f(a.y), hi_f(v.y) + hi_f(a.y)),
+                      pack2(lo_f(v.z) + lo_f(a.z), hi_f(v.z) + hi_f(a.z)),
+                      pack2(lo_f(v.w) + lo_f(a.w), hi_f(v.w) + hi_f(a.w)));
+}
+__device__ __forceinline__ float square_sum8(const uint4& v, float ss) {
+    const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = lo_f(u[i]), b = hi_f(u[i]);
+        ss = fmaf(a, a, ss);
+        ss = fmaf(b, b, ss);
+    }
+    return ss;
+}
+__device__ __forceinline__ uint4 scale8(const uint4& v, const uint4& g, float inv) {
+    return make_uint4(pack2(lo_f(v.x) * inv * lo_f(g.x), hi_f(v.x) * inv * hi_f(g.x)),
+                      pack2(lo_f(v.y) * inv * lo_f(g.y), hi_f(v.y) * inv * hi_f(g.y)),
+                      pack2(lo_f(v.z) * inv * lo_f(g.z), hi_f(v.z) * inv * hi_f(g.z)),
+                      pack2(lo_f(v.w) * inv * lo_f(g.w), hi_f(v.w) * inv * hi_f(g.w)));
+}
 __global__ void __launch_bounds__(kThreads)
     resnorm_kernel(uint16_t* __restrict__ res, const uint16_t* __restrict__ delta,
                    const uint16_t* __restrict__ w, uint16_t* __restrict__ out, uint32_t n,
@@ -179,36 +193,56 @@ __global__ void __launch_bounds__(kThreads)
     for (uint32_t c = threadIdx.x; c < n / 8u; c += kThreads) {
         uint4 v = ld16(r + 8u * c);
         if (d != nullptr) {
-            const uint4 a = ld16(d + 8u * c);
-            v.x = pack2(lo_f(v.x) + lo_f(a.x), hi_f(v.x) + hi_f(a.x));
-            v.y = pack2(lo_f(v.y) + lo_f(a.y), hi_f(v.y) + hi_f(a.y));
-            v.z = pack2(lo_f(v.z) + lo_f(a.z), hi_f(v.z) + hi_f(a.z));
-            v.w = pack2(lo_f(v.w) + lo_f(a.w), hi_f(v.w) + hi_f(a.w));
+            v = add8(v, ld16(d + 8u * c));
             *reinterpret_cast<uint4*>(r + 8u * c) = v;
         }
-        const uint32_t u[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float a = lo_f(u[i]), b = hi_f(u[i]);
-            ss = fmaf(a, a, ss);
-            ss = fmaf(b, b, ss);
-        }
+        ss = square_sum8(v, ss);
     }
     const float inv = 1.0f / sqrtf(block_sum(ss, s4) / (float)n + eps);
-    for (uint32_t c = threadIdx.x; c < n / 8u; c += kThreads) {
-        const uint4 v = ld16(r + 8u * c), g = ld16(w + 8u * c);
-        uint4 y;
-        y.x = pack2(lo_f(v.x) * inv * lo_f(g.x), hi_f(v.x) * inv * hi_f(g.x));
-        y.y = pack2(lo_f(v.y) * inv * lo_f(g.y), hi_f(v.y) * inv * hi_f(g.y));
-        y.z = pack2(lo_f(v.z) * inv * lo_f(g.z), hi_f(v.z) * inv * hi_f(g.z));
-        y.w = pack2(lo_f(v.w) * inv * lo_f(g.w), hi_f(v.w) * inv * hi_f(g.w));
-        *reinterpret_cast<uint4*>(o + 8u * c) = y;
-    }
+    for (uint32_t c = threadIdx.x; c < n / 8u; c += kThreads)
+        *reinterpret_cast<uint4*>(o + 8u * c) = scale8(ld16(r + 8u * c), ld16(w + 8u * c), inv);
 }
 
-__device__ __forceinline__ float silu_mul(float g, float u) {
-    return g / (1.0f + expf(-g)) * u;
+// The same for rows of 2048 whose addend comes as the fp32 sums of S K
+// splits, part[s][rows][2048] (gemm_tiles.hip): added in split order and
+// rounded to bf16 (the projection's output) before the residual add. A thread
+// holds its 8 elements throughout; every load is issued before the first use
+// (the splits are S x 8 KB per row against 4 KB of bf16: at 201 rows and 4
+// splits 1.4 us more than the bf16 form, where the split saves 7.6 us of the
+// down projection).
+template <uint32_t S>
+__global__ void __launch_bounds__(kThreads)
+    resnorm_splits_kernel(uint16_t* __restrict__ res, const float* __restrict__ part,
+                          const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
+                          float eps) {
+    constexpr uint32_t n = 8u * kThreads;
+    __shared__ float s4[4];
+    const size_t at = (size_t)blockIdx.x * n + 8u * threadIdx.x;
+    const size_t plane = (size_t)gridDim.x * n;
+    const uint4 r = ld16(res + at), g = ld16(w + 8u * threadIdx.x);
+    float4 p[S][2];
+#pragma unroll
+    for (uint32_t s = 0; s < S; ++s)
+#pragma unroll
+        for (uint32_t h = 0; h < 2u; ++h)
+            p[s][h] = *reinterpret_cast<const float4*>(part + s * plane + at + 4u * h);
+#pragma unroll
+    for (uint32_t s = 1; s < S; ++s)
+#pragma unroll
+        for (uint32_t h = 0; h < 2u; ++h) {
+            p[0][h].x += p[s][h].x;
+            p[0][h].y += p[s][h].y;
+            p[0][h].z += p[s][h].z;
+            p[0][h].w += p[s][h].w;
+        }
+    const uint4 d = make_uint4(pack2(p[0][0].x, p[0][0].y), pack2(p[0][0].z, p[0][0].w),
+                               pack2(p[0][1].x, p[0][1].y), pack2(p[0][1].z, p[0][1].w));
+    const uint4 v = add8(r, d);
+    *reinterpret_cast<uint4*>(res + at) = v;
+    const float inv = 1.0f / sqrtf(block_sum(square_sum8(v, 0.f), s4) / (float)n + eps);
+    *reinterpret_cast<uint4*>(out + at) = scale8(v, g, inv);
 }
+
 __device__ __forceinline__ uint4 swiglu8(const uint4& g, const uint4& u) {
     uint4 y;
     y.x = pack2(silu_mul(lo_f(g.x), lo_f(u.x)), silu_mul(hi_f(g.x), hi_f(u.x)));
@@ -500,7 +534,6 @@ __global__ void __launch_bounds__(64u * WV)
 // row is one weight load round and 16 FMAs per chunk. e4m3 -> fp32 is v_cvt_pk_f32_fp8 (exact); the codes S.1111.111,
 // which it reads as NaN, are decoded by the bit layout instead (+-480) in a
 // rarely taken branch, so every code has the meaning of the oracle's decoder.
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ float e4m3_bits_to_f32(uint32_t b) {
     // exponent field e, mantissa m: e = 0 -> m/8 * 2^-6, else (1 + m/8) 2^(e-7)
@@ -785,9 +818,7 @@ bool launch_gemv_m(uint32_t M, const GemvArgs& a, hipStream_t st) {
 // ---- row GEMM for prefill chunks of MC_MODEL_GEMM_ROWS_MIN..MAX rows ----
 // y[m][n] = bf16(sum_k W[n][k] x[m][k]) (or, SWI, bf16(silu(g) * u) of the
 // gate row n and up row N + n, each rounded to bf16 first, as the GEMV
-// epilogue) for 9..32 activation rows. The library kernels stream the
-// weights slowly at these sizes (hipBLASLt: a 32-row qkv projection in
-// 12 us, 0.85 TB/s); this kernel reads each weight byte once, at 1.1-3.8
+// epilogue) for 9..32 activation rows. The kernel reads each weight byte once, at 1.1-3.8
 // TB/s (5.3-7.7 us for qkv, 13-18 us for gate_up + SwiGLU at 9-32 rows).
 // Its activation reads grow with the rows, which bounds it above 32.
 // Workgroup = 4 waves (8 for K = 6144) on one 16-row block of W (two
@@ -942,6 +973,33 @@ extern "C" mc_status_t mc_model_rmsnorm_rows(uint16_t* d_res, const uint16_t* d_
     hipLaunchKernelGGL(resnorm_kernel, dim3(rows), dim3(kThreads), 0, (hipStream_t)stream, d_res,
                        d_add, d_weight, d_out, n, eps);
     return check_launch("rmsnorm launch failed");
+}
+
+extern "C" mc_status_t mc_model_rmsnorm_splits(uint16_t* d_res, const float* d_partials,
+                                               uint32_t splits, const uint16_t* d_weight,
+                                               uint16_t* d_out, uint32_t rows, float eps,
+                                               void* stream) {
+    TraceRange trace_range("mc_model_rmsnorm_splits");
+    if (d_res == nullptr || d_partials == nullptr || d_weight == nullptr || d_out == nullptr ||
+        rows == 0u || splits == 0u || splits > 8u || !(eps >= 0.f) ||
+        reinterpret_cast<uintptr_t>(d_partials) % 16u) {
+        set_error("mc_model_rmsnorm_splits: invalid args (rows=%u splits=%u eps=%g; splits 1..8, "
+                  "partials 16-byte aligned)",
+                  rows, splits, (double)eps);
+        return MC_E_INVALID_ARGUMENT;
+    }
+    hipStream_t st = (hipStream_t)stream;
+#define MC_SPLITS(S)                                                                            \
+    case S:                                                                                     \
+        hipLaunchKernelGGL((resnorm_splits_kernel<S>), dim3(rows), dim3(kThreads), 0, st, d_res, \
+                           d_partials, d_weight, d_out, eps);                                   \
+        break;
+    switch (splits) {
+        MC_SPLITS(1) MC_SPLITS(2) MC_SPLITS(3) MC_SPLITS(4)
+        MC_SPLITS(5) MC_SPLITS(6) MC_SPLITS(7) MC_SPLITS(8)
+    }
+#undef MC_SPLITS
+    return check_launch("rmsnorm (split sums) launch failed");
 }
 
 extern "C" mc_status_t mc_model_swiglu_rows(const uint16_t* d_src, uint16_t* d_out,

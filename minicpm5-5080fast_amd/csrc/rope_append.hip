@@ -137,6 +137,24 @@ __global__ void __launch_bounds__(256) rope_append_kernel(
     }
 }
 
+// (cos, sin) of the 64 rotate pairs of every token, as 128 floats in columns
+// kKCol.. of its qkv row: one wave per token. A prefill chunk writes them once
+// for all layers (the qkv projection's epilogue reads them; evaluated there
+// they would be evaluated for 18 heads per token and layer).
+__global__ void __launch_bounds__(256) rope_table_kernel(uint16_t* __restrict__ qkv,
+                                                         uint32_t tokens,
+                                                         const uint32_t* __restrict__ d_base_pos,
+                                                         float theta,
+                                                         const float* __restrict__ inv_freq) {
+    const uint32_t t = blockIdx.x * kWaves + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    if (t >= tokens) return;
+    const float f = inv_freq != nullptr ? inv_freq[lane]
+                                        : (float)pow((double)theta, -(double)lane / 64.0);
+    float c, s;
+    rope_sincos((float)(*d_base_pos + t) * f, &c, &s);
+    reinterpret_cast<float2*>(qkv + (size_t)t * kRow + kKCol)[lane] = make_float2(c, s);
+}
+
 __global__ void inv_freq_init_kernel(float* __restrict__ table, double theta) {
     const uint32_t p = threadIdx.x;
     if (p < 64u) table[p] = (float)pow(theta, -(double)p / 64.0);
@@ -180,4 +198,19 @@ extern "C" mc_status_t mc_kv_rope_append(uint16_t* d_qkv, uint32_t tokens,
                        (hipStream_t)stream, d_qkv, tokens, d_base_pos, layer,
                        d_page_table, d_kv_pool, ly, (float)rope_theta, d_inv_freq);
     return mckv::check_launch("rope_append launch failed");
+}
+
+extern "C" mc_status_t mc_kv_rope_table(uint16_t* d_qkv, uint32_t tokens,
+                                        const uint32_t* d_base_pos, double rope_theta,
+                                        const float* d_inv_freq, void* stream) {
+    mckv::TraceRange trace_range("mc_kv_rope_table");
+    if (d_qkv == nullptr || reinterpret_cast<uintptr_t>(d_qkv) % 16u != 0u ||
+        d_base_pos == nullptr || tokens == 0 || (d_inv_freq == nullptr && !(rope_theta > 0.0))) {
+        mckv::set_error("mc_kv_rope_table: invalid args (tokens=%u)", tokens);
+        return MC_E_INVALID_ARGUMENT;
+    }
+    hipLaunchKernelGGL(mckv::rope_table_kernel, dim3((tokens + mckv::kWaves - 1u) / mckv::kWaves),
+                       dim3(256), 0, (hipStream_t)stream, d_qkv, tokens, d_base_pos,
+                       (float)rope_theta, d_inv_freq);
+    return mckv::check_launch("rope table launch failed");
 }
