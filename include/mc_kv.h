@@ -344,14 +344,18 @@ mc_status_t mc_debug_batch_group_stats(mc_batch_group_t group, uint64_t* steps,
 int mc_debug_batch_breakdown_collect(mc_batch_group_t group, double* out_ms, int n);
 
 /* Prefill workgroup shape: 0 = 32 query rows on 8 waves, 1 = 16 rows on 4
- * waves, 2 = 16 rows on two 4-wave halves taking alternate key steps, 3 and
- * 4 = 8 and 4 rows on four key sets taking alternate 32-key blocks,
+ * waves, 2 = 16 rows on two 4-wave halves taking alternate key steps,
  * 0xFFFFFFFF = chosen per launch (default). All compute the same softmax;
  * shapes differ in tile boundaries (key splits) and summation order, within
  * the attention tolerance. The previous value is stored to *previous when
  * that is not NULL. Process-wide; for tests that run every shape. No
  * reference counterpart. */
 mc_status_t mc_kv_debug_prefill_shape(uint32_t shape, uint32_t* previous);
+
+/* Key-set prefill workgroups (4 or 8 query rows, four key sets taking alternate
+ * 32-key blocks): rows = 4 or 8 runs every launch on them, before the hook
+ * above; 0 = chosen per launch (default). Otherwise as above. */
+mc_status_t mc_kv_debug_prefill_key_sets(uint32_t rows, uint32_t* previous);
 
 /* Prefill job packing: with key splits off, two to three 32-row jobs per CU
  * and a prefix of at least T/4, one workgroup per CU runs a fixed 2-3 job

@@ -80,9 +80,11 @@ constexpr uint32_t kSetsRows = 1024u, kSetsSplitRows = 384u;
 // g_barrier_timeouts (read by mc_kv_debug_prefill_status).
 constexpr uint32_t kHalfBarrierSpins = 1u << 22;
 __device__ uint32_t g_barrier_timeouts;
-// Forced shape (debug hook; kAutoShape = chosen per launch) and job packing.
+// Forced shape and key-set rows (debug hooks; kAutoShape and 0 = chosen per
+// launch) and job packing.
 constexpr uint32_t kAutoShape = 0xFFFFFFFFu;
 std::atomic<uint32_t> g_shape{kAutoShape};
+std::atomic<uint32_t> g_key_sets{0u};
 std::atomic<uint32_t> g_packing{1u};
 
 // Compute units of the current device (cached per device; 0 if unknown).
@@ -944,11 +946,21 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(
 using namespace mckv;
 
 extern "C" mc_status_t mc_kv_debug_prefill_shape(uint32_t shape, uint32_t* previous) {
-    if (shape > mckv::kSets4 && shape != mckv::kAutoShape) {
-        set_error("mc_kv_debug_prefill_shape: shape %u is not 0..4 or 0xFFFFFFFF", shape);
+    if (shape > mckv::kHalves16 && shape != mckv::kAutoShape) {
+        set_error("mc_kv_debug_prefill_shape: shape %u is not 0, 1, 2 or 0xFFFFFFFF", shape);
         return MC_E_INVALID_ARGUMENT;
     }
     const uint32_t prev = mckv::g_shape.exchange(shape);
+    if (previous != nullptr) *previous = prev;
+    return MC_OK;
+}
+
+extern "C" mc_status_t mc_kv_debug_prefill_key_sets(uint32_t rows, uint32_t* previous) {
+    if (rows != 0u && rows != 4u && rows != 8u) {
+        set_error("mc_kv_debug_prefill_key_sets: rows %u is not 0, 4 or 8", rows);
+        return MC_E_INVALID_ARGUMENT;
+    }
+    const uint32_t prev = mckv::g_key_sets.exchange(rows);
     if (previous != nullptr) *previous = prev;
     return MC_OK;
 }
@@ -1062,6 +1074,8 @@ mc_status_t prefill_attention(const uint16_t* d_q_rows, uint32_t tokens,
     const uint32_t jobs8 = kHkv * ((tokens + 7u) / 8u), jobs4 = kHkv * ((tokens + 3u) / 4u);
     const uint32_t cus = cu_count(), cu = cus ? cus : 256u;
     uint32_t shape = g_shape.load(std::memory_order_relaxed);
+    if (const uint32_t rows = g_key_sets.load(std::memory_order_relaxed); rows != 0u)
+        shape = rows == 4u ? kSets4 : kSets8;
     if (shape == kAutoShape) {
         const bool short_prefix = keys != 0u && keys / 2u <= tokens;
         if (tokens <= (S_kv > 1u ? kSetsSplitRows : short_prefix ? 2u * kSetsRows : kSetsRows)) {

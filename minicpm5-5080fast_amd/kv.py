@@ -159,11 +159,19 @@ PREFILL_SHAPE_AUTO = 0xFFFFFFFF
 
 def debug_prefill_shape(shape: int) -> int:
     """Forces the prefill workgroup shape (0 = 32 rows, 1 = 16 rows on 4
-    waves, 2 = 16 rows on two halves, 3 / 4 = 8 / 4 rows on four key sets,
-    PREFILL_SHAPE_AUTO = per launch) and returns the previous setting. Debug
-    hook, no reference counterpart."""
+    waves, 2 = 16 rows on two halves, PREFILL_SHAPE_AUTO = per launch) and
+    returns the previous setting. Debug hook, no reference counterpart."""
     prev = C.c_uint32(0)
     check(lib().mc_kv_debug_prefill_shape(shape, C.byref(prev)), "debug_prefill_shape")
+    return prev.value
+
+
+def debug_prefill_key_sets(rows: int) -> int:
+    """Forces the key-set prefill workgroups of 4 or 8 query rows (0 = chosen
+    per launch) and returns the previous setting. Debug hook, no reference
+    counterpart."""
+    prev = C.c_uint32(0)
+    check(lib().mc_kv_debug_prefill_key_sets(rows, C.byref(prev)), "debug_prefill_key_sets")
     return prev.value
 
 

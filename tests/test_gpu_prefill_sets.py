@@ -8,11 +8,11 @@ from test_gpu_prefill import barrier_status_clear, run_prefill  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(params=[3, 4], ids=["rows8", "rows4"])
+@pytest.fixture(params=[8, 4], ids=["rows8", "rows4"])
 def shape(kvm, request):
-    prev = kvm.debug_prefill_shape(request.param)
+    prev = kvm.debug_prefill_key_sets(request.param)
     yield request.param
-    kvm.debug_prefill_shape(prev)
+    kvm.debug_prefill_key_sets(prev)
 
 
 @pytest.mark.parametrize("T,base", [(1, 0), (3, 0), (4, 28), (5, 31), (7, 32), (8, 120), (9, 127),
