@@ -113,21 +113,12 @@ mc_status_t gemm_bf16(const Forward& f, const uint16_t* x, uint32_t M, const uin
 // or splits = 0 for rocBLAS (MC_PREFILL_GEMM_DEFAULT=1 sends all there).
 struct PrefillPlan {
     GemmPlan qkv, o, gate_up, down;
-    bool rope = false;  // qkv's tiles rotate and append (no RoPE kernel)
 };
 PrefillPlan prefill_plan(const Forward& f, uint32_t n) {
     PrefillPlan p;
     if (gemm_defaults_only() || n <= MC_MODEL_GEMM_ROWS_MAX) return p;
     p.gate_up = gemm_tiles_plan(n, kInter, kHidden, TileEnd::kSwiglu, 1u, 1u);
-    // The rope form saves the RoPE kernel (3.5 us and 2.4 ns per row with its
-    // launch gap) but not every shape takes it.
-    float plain_us, rope_us;
-    p.qkv = gemm_tiles_plan(n, kQkvCols, kHidden, TileEnd::kPlain, 1u, 1u, &plain_us);
-    const GemmPlan r = gemm_tiles_plan(n, kQkvCols, kHidden, TileEnd::kRope, 1u, 1u, &rope_us);
-    if (rope_us < plain_us + 3.5f + 0.0024f * (float)n) {
-        p.qkv = r;
-        p.rope = true;
-    }
+    p.qkv = gemm_tiles_plan(n, kQkvCols, kHidden, TileEnd::kRope, 1u, 1u);
     // the split sums [splits][n][kHidden] fp32 lie in the gate_up buffer of
     // f.rows rows of 2 kInter bf16
     const uint32_t fit = (uint32_t)((size_t)f.rows * 2u * kInter * 2u / ((size_t)n * kHidden * 4u));
@@ -445,7 +436,8 @@ mc_status_t forward_prefill(const Forward& f, const int32_t* d_ids, uint32_t n, 
         set_error("forward_prefill: invalid KV layout");
         return MC_E_INTERNAL;
     }
-    if (plan.rope) FWD_OR_RETURN(mc_kv_rope_table(f.qkv, n, f.d_seq_len, kTheta, inv_freq, st));
+    if (plan.qkv.splits != 0u)
+        FWD_OR_RETURN(mc_kv_rope_table(f.qkv, n, f.d_seq_len, kTheta, inv_freq, st));
     auto proj = [&](const uint16_t* x, const uint16_t* W, uint32_t N, uint32_t K, uint16_t* y,
                     const GemmPlan& p) {
         if (rows) return mc_model_gemm_rows(W, x, K, y, N, n, N, K, 0u, st);
@@ -471,7 +463,7 @@ mc_status_t forward_prefill(const Forward& f, const int32_t* d_ids, uint32_t n, 
     for (uint32_t l = 0; l < kModelLayers; ++l) {
         if (layer_dump)
             FWD_OR_RETURN(dump_bf16(dump_name("layer", l, "hidden_in.f32"), res_last, kHidden, st));
-        if (plan.rope) {
+        if (plan.qkv.splits != 0u) {  // rotates and appends as its epilogue
             FWD_OR_RETURN(gemm_tiles({f.normed, w.qkv[l], f.qkv, nullptr, n, kQkvCols, kHidden,
                                       false, {f.d_seq_len, f.d_pt, f.pool, ly, l, 0u}},
                                      plan.qkv, st));

@@ -34,9 +34,10 @@
 //
 // Epilogues: the SwiGLU saves 12.7 us per layer at 2048 rows and 50 at 8448;
 // the qkv projection's RoPE and K/V append saves the RoPE kernel and its
-// launch (whole prompts: 64 tokens 2.67 -> 2.42 ms, 201 3.27 -> 3.06, 1500
+// launch (whole prompts: 64 tokens 2.67 -> 2.31 ms, 201 3.27 -> 2.98, 1500
 // 9.4 -> 8.8, 8448 44.3 -> 44.0); its cos / sin come from a table written once
-// per chunk.
+// per chunk. Loading all of a tile's cos / sin before the rotations was no
+// faster than row by row.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -77,6 +78,13 @@ __device__ __forceinline__ uint32_t block_row(uint32_t b, uint32_t nb, uint32_t 
     return (b | 1u) < nb ? 32u * (b >> 1) + 8u * (p >> 2) + 4u * (b & 1u) + (p & 3u) : 16u * b + p;
 }
 
+// Pool row of the token in row m.
+__device__ __forceinline__ uint16_t* rope_slot(const RopeAppend& r, uint32_t m) {
+    const uint32_t pos = *r.base_pos + r.row0 + m;
+    const uint32_t page = clamp_page(r.ly, r.page_table[table_index(r.ly, pos)]);
+    return r.pool + token_base(r.ly, r.layer, page, pos & r.ly.pmask);
+}
+
 // grid = one workgroup per (m tile, n tile, K split). Workgroup i runs on XCD
 // i mod 8: each XCD takes one contiguous range of tiles, numbered within
 // groups of `group` m tiles with m fastest, so the workgroups sharing a W
@@ -84,8 +92,9 @@ __device__ __forceinline__ uint32_t block_row(uint32_t b, uint32_t nb, uint32_t 
 // SWI: 16-row blocks of gate rows alternate with the blocks of the up rows N
 // below them (w is [2N][K]); y[m][n] = bf16(silu(bf16 g) * bf16 u).
 // ROPE: blocks of a head's dims 0..63 alternate with the blocks of the dims 64
-// above them; m tiles and columns count dim pairs (N / 2), and the pair is
-// rotated in fp32 from its bf16 projections as in rope_append.hip.
+// above them (a wave of one block: 8 rows of each in it); columns count dim
+// pairs (N / 2), and the pair is rotated in fp32 from its bf16 projections as
+// in rope_append.hip.
 // Otherwise y (part == nullptr), or the fp32 sums of this K split in
 // part[split][M][N].
 template <uint32_t BM, uint32_t BN, uint32_t WM, uint32_t WN, uint32_t ST, uint32_t BK,
@@ -105,7 +114,8 @@ __global__ void __launch_bounds__(64u * WM * WN)
     constexpr uint32_t TM = BM / WM, TN = BN / WN, MB = TM / 16u, NB = TN / 16u;
     static_assert(ROWS % (RPI * NW) == 0u && BM % RPI == 0u, "whole loads per wave");
     static_assert(NS % 2u == 0u, "operand register sets alternate per substep");
-    static_assert(!PAIR || NB % 2u == 0u, "a wave holds both blocks of a pair");
+    constexpr bool HALVES = ROPE && NB == 1u;  // a block holds 8 pairs: lo rows, hi rows
+    static_assert(!PAIR || NB % 2u == 0u || HALVES, "a wave holds both sides of a pair");
     static_assert(ST * ROWS * BK * 2u <= 160u * 1024u, "LDS");
     __shared__ __align__(1024) uint16_t lds[ST][ROWS * BK];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -139,7 +149,10 @@ __global__ void __launch_bounds__(64u * WM * WN)
             if constexpr (SWI)
                 row = min(n0 + wq * (TN / 2u) + block_row(b >> 1, NB / 2u, p), N - 1u) +
                       ((b & 1u) ? N : 0u);
-            else if constexpr (ROPE) {
+            else if constexpr (HALVES) {
+                const uint32_t f = min(n0 + wq * 8u + (p & 7u), N / 2u - 1u);
+                row = (f >> 6) * kD + (f & 63u) + (p >= 8u ? 64u : 0u);
+            } else if constexpr (ROPE) {
                 const uint32_t f =
                     min(n0 + wq * (TN / 2u) + block_row(b >> 1, NB / 2u, p), N / 2u - 1u);
                 row = (f >> 6) * kD + (f & 63u) + ((b & 1u) ? 64u : 0u);
@@ -232,8 +245,36 @@ __global__ void __launch_bounds__(64u * WM * WN)
 #pragma unroll
     for (uint32_t j = 0; j < MB; ++j) {
         const uint32_t m = m0 + wm * TM + 16u * j + col;
+        if constexpr (HALVES) {
+            // lanes < 32 hold the lower dims, the lane 32 above the dims + 64
+            const uint32_t f = n0 + wn * 8u + 4u * (grp & 1u), d = f & 63u;
+            const uint32_t up = grp >> 1, lo_col = (f >> 6) * kD + d;
+            float lo[4], hi[4], o[4];
+#pragma unroll
+            for (uint32_t v = 0; v < 4u; ++v) {
+                const uint32_t u = __float_as_uint(round_bf16(acc[0][j][v]));
+                const auto h = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+                lo[v] = __uint_as_float(h[0]);
+                hi[v] = __uint_as_float(h[1]);
+                o[v] = up ? hi[v] : lo[v];
+            }
+            if (m >= M || f >= N / 2u) continue;
+            uint16_t* yr = y + (size_t)m * N;
+            if (lo_col < kVCol) {  // q, k: rotate
+                const float2* cs = reinterpret_cast<const float2*>(yr + kKCol) + d;
+#pragma unroll
+                for (uint32_t v = 0; v < 4u; ++v)
+                    o[v] = up ? rope_rotate(hi[v], lo[v], cs[v].x, cs[v].y, false)
+                              : rope_rotate(lo[v], hi[v], cs[v].x, cs[v].y, true);
+            }
+            uint16_t* dst = yr + lo_col;
+            if (lo_col >= kKCol) dst = rope_slot(rope, m) + (lo_col - kKCol);
+            *reinterpret_cast<uint2*>(dst + 64u * up) =
+                make_uint2(pack2(o[0], o[1]), pack2(o[2], o[3]));
+            continue;
+        }
         if (m >= M) continue;
-        if constexpr (ROPE) {
+        if constexpr (ROPE && !HALVES) {
             uint16_t* yr = y + (size_t)m * N;
             const float2* cs = reinterpret_cast<const float2*>(yr + kKCol);
             uint16_t* slot = nullptr;  // the token's page row, for k / v heads
@@ -263,13 +304,7 @@ __global__ void __launch_bounds__(64u * WM * WN)
                 }
                 uint16_t* o = yr + lo_col;
                 if (lo_col >= kKCol) {
-                    if (slot == nullptr) {
-                        const uint32_t pos = *rope.base_pos + rope.row0 + m;
-                        const uint32_t page =
-                            clamp_page(rope.ly, rope.page_table[table_index(rope.ly, pos)]);
-                        slot = rope.pool +
-                               token_base(rope.ly, rope.layer, page, pos & rope.ly.pmask);
-                    }
+                    if (slot == nullptr) slot = rope_slot(rope, m);
                     o = slot + (lo_col - kKCol);
                 }
                 if (two) {
@@ -352,13 +387,13 @@ struct TileCost {
 };
 struct TileShape {
     uint16_t bm, bn, bk;
-    bool rope;  // waves hold W blocks in pairs: takes the rope form
+    bool rope;  // waves hold one W block, or blocks in pairs: takes the rope form
     TileCost plain, swiglu;
 };
 constexpr TileShape kShapes[] = {
-    {32, 64, 128, false, {3.92f, 0.00f, 0.166f}, {}},
-    {48, 64, 128, false, {2.46f, 1.52f, 0.190f}, {}},
-    {64, 64, 128, false, {2.54f, 1.78f, 0.215f}, {}},
+    {32, 64, 128, true, {3.92f, 0.00f, 0.166f}, {}},
+    {48, 64, 128, true, {2.46f, 1.52f, 0.190f}, {}},
+    {64, 64, 128, true, {2.54f, 1.78f, 0.215f}, {}},
     {64, 64, 64, false, {}, {9.06f, 0.00f, 0.195f}},
     {64, 96, 64, false, {}, {9.17f, 0.00f, 0.255f}},
     {96, 64, 64, true, {3.89f, 0.76f, 0.243f}, {8.89f, 0.00f, 0.238f}},

@@ -138,7 +138,8 @@ def test_norm_of_split_sums(lib, orc, dev, splits):
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
 
 
-@pytest.mark.parametrize("shape", [5, 6, 7, 8, 10, 11, 12, 13, 15, 16, 17, AUTO])
+@pytest.mark.parametrize("shape", [0, 1, 2, 5, 6, 7, 8, 10, 11, 12, 13, 15, 16, 17,
+                                   AUTO])
 def test_rope_form(lib, pkg, orc, dev, shape):
     """mc_model_gemm_tiles_rope equals the plain tiles followed by
     mc_kv_rope_append bit for bit (q columns and every page slot), for whole
@@ -197,6 +198,6 @@ def test_rejects_bad_arguments(lib, pkg, dev):
     g = lib.mc_model_gemm_tiles_rope
     for a in ((p, p, p, 0, 128, p, 0, p, p, lay, AUTO), (p, p, p, 8, 192, p, 0, p, p, lay, AUTO),
               (p, p, p, 8, 128, p, 2, p, p, lay, AUTO), (p, p, p, 8, 128, p, 0, None, p, lay, AUTO),
-              (p, p, odd, 8, 128, p, 0, p, p, lay, AUTO), (p, p, p, 8, 128, p, 0, p, p, lay, 0)):
+              (p, p, odd, 8, 128, p, 0, p, p, lay, AUTO), (p, p, p, 8, 128, p, 0, p, p, lay, 14)):
         assert g(*a, stream()) == 1, a[3:]
     assert lib.mc_kv_rope_table(p, 0, p, 5e6, None, stream()) == 1
