@@ -24,6 +24,8 @@
 // states in LDS (no key splits, at most two tiles per CU: the heaviest
 // causal tile sets the time; each half waits only for its own waves, so the
 // halves run out of phase), else as 256-thread workgroups two per CU.
+// Chunks of up to about a thousand rows run 4- or 8-row workgroups with four
+// key sets instead (prefill_sets_kernel).
 // The 32 rows x 8 query heads of a KV head are 256 query vectors: wave w owns
 // two 16-column groups, group g holding rows 4w + 2g + {0, 1} x heads 0..7.
 // Keys stream in 64-position steps gathered through the page table into LDS
