@@ -357,6 +357,14 @@ mc_status_t mc_kv_debug_prefill_shape(uint32_t shape, uint32_t* previous);
  * above; 0 = chosen per launch (default). Otherwise as above. */
 mc_status_t mc_kv_debug_prefill_key_sets(uint32_t rows, uint32_t* previous);
 
+/* The workgroup shape (0..2 as above, 3 / 4: key sets of 8 / 4 rows) and key
+ * splits that a prefill attention of `tokens` rows with at most S_kv splits
+ * takes on 256 CUs when nothing is forced; keys: those its last row attends
+ * where the caller knows them (0: not known, as for mc_kv_attention_prefill).
+ * Host only. No reference counterpart. */
+mc_status_t mc_kv_debug_prefill_choice(uint32_t tokens, uint32_t S_kv, uint32_t keys,
+                                       uint32_t* shape, uint32_t* splits);
+
 /* Prefill job packing: with key splits off, two to three 32-row jobs per CU
  * and a prefix of at least T/4, one workgroup per CU runs a fixed 2-3 job
  * packing instead of greedy dispatch (identical results). enable = 0 turns it

@@ -73,6 +73,7 @@ _SIGS = {
     "mc_kv_batch_advance": (C.c_int, [_P, _P, _P, _u32, _P]),
     "mc_kv_debug_prefill_shape": (C.c_int, [_u32, _P]),
     "mc_kv_debug_prefill_key_sets": (C.c_int, [_u32, _P]),
+    "mc_kv_debug_prefill_choice": (C.c_int, [_u32, _u32, _u32, C.POINTER(_u32), C.POINTER(_u32)]),
     "mc_kv_debug_prefill_packing": (C.c_int, [_u32, _P]),
     "mc_kv_debug_prefill_status": (C.c_int, [_P, _u32]),
     "mc_kv_debug_prefill_force_timeouts": (C.c_int, [_u32]),

@@ -74,8 +74,11 @@ constexpr uint32_t kRows32 = 0u, kRows16 = 1u, kHalves16 = 2u, kSets8 = 3u, kSet
 // 32-row workgroup count (2 per CU) below which the 16-row shapes are used.
 constexpr uint32_t kSmallBelow = 512u;
 // Rows up to which a launch without / with key splits runs on the key-set
-// workgroups (the reasons stand at the choice below).
-constexpr uint32_t kSetsRows = 1024u, kSetsSplitRows = 384u;
+// workgroups, and with splits the fewest splits that must fit at one workgroup
+// per CU, or the most keys per such split (the reasons stand at
+// prefill_choice).
+constexpr uint32_t kSetsRows = 1024u, kSetsSplitRows = 384u, kSetsSplits = 5u;
+constexpr uint32_t kSetsSplitKeys = 1200u;
 // Polls of a per-half barrier before it gives up (s_sleep 1 = 64 clocks each,
 // about 2^22 * 64 / 2.4 GHz = 0.1 s): far beyond any legal wait, so it only
 // ends a wait that can never complete. A timed-out wait is counted in
@@ -942,6 +945,58 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(
         (uint32_t)a | ((uint32_t)b << 16);
 }
 
+// Workgroup shape and key splits of a launch of `tokens` rows with at most
+// S_kv splits on `cu` CUs; keys: those the last row attends, 0 = not known.
+// The key-set workgroups: 4 rows each while that gives every CU at most one,
+// else 8 (us per layer at base 0: 512 rows 11.0 with 4 rows, 13.2 with 8; 1024
+// rows 21.2 / 19.5).
+// * S_kv = 1: to kSetsRows rows (8 rows against the halves below: 1024 rows
+//   19.5 / 27.5, at base 8000 109 / 152), and to twice as many where the prefix
+//   is known to be no longer than the chunk (1500 rows 25.4 / 35.5, but 107 /
+//   100 at base 4000, where two rounds of workgroups pack worse).
+// * S_kv > 1 is the most key splits. Every 8-row workgroup reads the whole
+//   prefix, where a 16-row tile reads it once for twice the rows, so key sets
+//   pay while the chunk is short: with as many splits as keep one workgroup per
+//   CU (256 rows at base 2000: 20.9 with 2 splits, 24.6 with 8), up to
+//   kSetsSplits of them fit (200 rows with 8 splits asked for, K/V from HBM,
+//   16-row tiles in parentheses: base 0 14.5 (13.7), 4000 23.8 (27.8), 30000
+//   101 (107), 120000 363 (393)). With fewer, to kSetsSplitRows rows where the
+//   keys are known to be at most kSetsSplitKeys per split (256 rows at base
+//   4000 25.3 (29.5), at 30000 123 (110); 384 rows at base 1000 20.7 (23.0), at
+//   4000 39.1 (33.8), at 30000 226 (135)). Longer chunks keep 16-row tiles and
+//   all splits (777 rows at base 3001: 42.4 with 5 splits, key sets 49.7; at
+//   base 0 they would take 16.8 against 25.0, so a caller that knows its base
+//   passes S_kv = 1 there).
+// Above, 32-row tiles while they give at least two workgroups per CU, and
+// 16-row tiles below that, as two halves on alternate key steps when the
+// launch has no key splits and at most two 16-row jobs per CU (the
+// heaviest causal tile then sets the time, and the halves take it at
+// twice the rate), else as 4-wave workgroups two per CU. Measured
+// (base 0): T=3072 65.2 us with halves against 69.3, T=4096 125 (32 rows)
+// -> 118 -> 99.7 us; T=6144 178.5 us with 4-wave workgroups against
+// 210 with halves. With S_kv > 1 a tile's split boundaries follow its
+// last row, so they differ between tile heights.
+struct PrefillChoice {
+    uint32_t shape, splits;
+};
+PrefillChoice prefill_choice(uint32_t tokens, uint32_t S_kv, uint32_t keys, uint32_t cu) {
+    const uint32_t ntq32 = (tokens + 31u) / 32u, ntq16 = (tokens + 15u) / 16u;
+    const uint32_t jobs8 = kHkv * ((tokens + 7u) / 8u), jobs4 = kHkv * ((tokens + 3u) / 4u);
+    const uint32_t s4 = std::min(S_kv, cu / jobs4), s8 = std::min(S_kv, cu / jobs8);
+    const bool short_prefix = keys != 0u && keys / 2u <= tokens;
+    bool sets = tokens <= (short_prefix ? 2u * kSetsRows : kSetsRows);
+    if (S_kv > 1u)
+        sets = tokens <= kSetsSplitRows &&
+               (s8 >= std::min(S_kv, kSetsSplits) || (keys != 0u && keys <= kSetsSplitKeys * s8));
+    if (sets) {
+        const bool rows4 = s4 >= 1u && s4 >= s8;
+        return {rows4 ? kSets4 : kSets8, std::max(1u, rows4 ? s4 : s8)};
+    }
+    if (kHkv * ntq32 * S_kv >= kSmallBelow) return {kRows32, S_kv};
+    if (S_kv == 1u && kHkv * ntq16 <= 2u * cu) return {kHalves16, 1u};
+    return {kRows16, S_kv};
+}
+
 }  // namespace
 }  // namespace mckv
 
@@ -964,6 +1019,18 @@ extern "C" mc_status_t mc_kv_debug_prefill_key_sets(uint32_t rows, uint32_t* pre
     }
     const uint32_t prev = mckv::g_key_sets.exchange(rows);
     if (previous != nullptr) *previous = prev;
+    return MC_OK;
+}
+
+extern "C" mc_status_t mc_kv_debug_prefill_choice(uint32_t tokens, uint32_t S_kv, uint32_t keys,
+                                                  uint32_t* shape, uint32_t* splits) {
+    if (tokens == 0u || S_kv == 0u || S_kv > 8u || shape == nullptr || splits == nullptr) {
+        set_error("mc_kv_debug_prefill_choice: invalid args (tokens=%u S_kv=%u)", tokens, S_kv);
+        return MC_E_INVALID_ARGUMENT;
+    }
+    const PrefillChoice c = prefill_choice(tokens, S_kv, keys, 256u);
+    *shape = c.shape;
+    *splits = c.splits;
     return MC_OK;
 }
 
@@ -1049,48 +1116,15 @@ mc_status_t prefill_attention(const uint16_t* d_q_rows, uint32_t tokens,
         return MC_E_INVALID_ARGUMENT;
     }
     hipStream_t st = (hipStream_t)stream;
-    // Shape. The key-set workgroups: 4 rows each while that gives every CU at
-    // most one, else 8 (us per layer at base 0: 512 rows 11.0 with 4 rows,
-    // 13.2 with 8; 1024 rows 21.2 / 19.5).
-    // * S_kv = 1: to kSetsRows rows (8 rows against the halves below: 1024
-    //   rows 19.5 / 27.5, at base 8000 109 / 152), and to twice as many where
-    //   the caller knows that the prefix is no longer than the chunk (1500
-    //   rows 25.4 / 35.5, but 107 / 100 at base 4000, where two rounds of
-    //   workgroups pack worse).
-    // * S_kv > 1 is the most key splits: to kSetsSplitRows rows the key sets,
-    //   with no more splits than keep one workgroup per CU (256 rows at base
-    //   2000: 20.9 with 2 splits, 24.6 with 8; 16-row tiles with 8: 23.7).
-    //   Longer chunks keep 16-row tiles and all splits (777 rows at base 3001:
-    //   42.4 with 5 splits, key sets 49.7; at base 0 they would take 16.8
-    //   against 25.0, so a caller that knows its base passes S_kv = 1 there).
-    // Above, 32-row tiles while they give at least two workgroups per CU, and
-    // 16-row tiles below that, as two halves on alternate key steps when the
-    // launch has no key splits and at most two 16-row jobs per CU (the
-    // heaviest causal tile then sets the time, and the halves take it at
-    // twice the rate), else as 4-wave workgroups two per CU. Measured
-    // (base 0): T=3072 65.2 us with halves against 69.3, T=4096 125 (32 rows)
-    // -> 118 -> 99.7 us; T=6144 178.5 us with 4-wave workgroups against
-    // 210 with halves. With S_kv > 1 a tile's split boundaries follow its
-    // last row, so they differ between tile heights.
-    const uint32_t ntq32 = (tokens + 31u) / 32u, ntq16 = (tokens + 15u) / 16u;
+    const uint32_t cus = cu_count();
     const uint32_t jobs8 = kHkv * ((tokens + 7u) / 8u), jobs4 = kHkv * ((tokens + 3u) / 4u);
-    const uint32_t cus = cu_count(), cu = cus ? cus : 256u;
     uint32_t shape = g_shape.load(std::memory_order_relaxed);
     if (const uint32_t rows = g_key_sets.load(std::memory_order_relaxed); rows != 0u)
         shape = rows == 4u ? kSets4 : kSets8;
     if (shape == kAutoShape) {
-        const bool short_prefix = keys != 0u && keys / 2u <= tokens;
-        if (tokens <= (S_kv > 1u ? kSetsSplitRows : short_prefix ? 2u * kSetsRows : kSetsRows)) {
-            const uint32_t s4 = std::min(S_kv, cu / jobs4), s8 = std::min(S_kv, cu / jobs8);
-            shape = s4 >= 1u && s4 >= s8 ? kSets4 : kSets8;
-            S_kv = std::max(1u, shape == kSets4 ? s4 : s8);
-        } else if (kHkv * ntq32 * S_kv >= kSmallBelow) {
-            shape = kRows32;
-        } else if (S_kv == 1u && kHkv * ntq16 <= 2u * cu) {
-            shape = kHalves16;
-        } else {
-            shape = kRows16;
-        }
+        const PrefillChoice c = prefill_choice(tokens, S_kv, keys, cus ? cus : 256u);
+        shape = c.shape;
+        S_kv = c.splits;
     }
 #define MC_PF_LAUNCH(PG, SM)                                                                 \
     hipLaunchKernelGGL((prefill_attn_kernel<PG, SM>),                                        \

@@ -175,6 +175,15 @@ def debug_prefill_key_sets(rows: int) -> int:
     return prev.value
 
 
+def debug_prefill_choice(tokens: int, splits: int, keys: int = 0) -> tuple[int, int]:
+    """(shape, key splits) that a prefill attention launch takes on 256 CUs;
+    keys = 0: not known to the launch. Debug hook, no reference counterpart."""
+    shape, s = C.c_uint32(0), C.c_uint32(0)
+    check(lib().mc_kv_debug_prefill_choice(tokens, splits, keys, C.byref(shape), C.byref(s)),
+          "debug_prefill_choice")
+    return shape.value, s.value
+
+
 def debug_prefill_packing(enable: bool) -> bool:
     """Turns the fixed prefill job packing on or off and returns the previous
     setting. Debug hook, no reference counterpart."""
