@@ -79,6 +79,9 @@ constexpr uint32_t kSmallBelow = 512u;
 // prefill_choice).
 constexpr uint32_t kSetsRows = 1024u, kSetsSplitRows = 384u, kSetsSplits = 5u;
 constexpr uint32_t kSetsSplitKeys = 1200u;
+// Keys known: fewest per split, and the most with which 1025..2048 rows run on
+// the key-set workgroups.
+constexpr uint32_t kSplitKeysMin = 512u, kSetsKeys = 2200u;
 // Polls of a per-half barrier before it gives up (s_sleep 1 = 64 clocks each,
 // about 2^22 * 64 / 2.4 GHz = 0.1 s): far beyond any legal wait, so it only
 // ends a wait that can never complete. A timed-out wait is counted in
@@ -951,9 +954,7 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(
 // else 8 (us per layer at base 0: 512 rows 11.0 with 4 rows, 13.2 with 8; 1024
 // rows 21.2 / 19.5).
 // * S_kv = 1: to kSetsRows rows (8 rows against the halves below: 1024 rows
-//   19.5 / 27.5, at base 8000 109 / 152), and to twice as many where the prefix
-//   is known to be no longer than the chunk (1500 rows 25.4 / 35.5, but 107 /
-//   100 at base 4000, where two rounds of workgroups pack worse).
+//   19.5 / 27.5, at base 8000 109 / 152).
 // * S_kv > 1 is the most key splits. Every 8-row workgroup reads the whole
 //   prefix, where a 16-row tile reads it once for twice the rows, so key sets
 //   pay while the chunk is short: with as many splits as keep one workgroup per
@@ -965,8 +966,21 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(
 //   4000 25.3 (29.5), at 30000 123 (110); 384 rows at base 1000 20.7 (23.0), at
 //   4000 39.1 (33.8), at 30000 226 (135)). Longer chunks keep 16-row tiles and
 //   all splits (777 rows at base 3001: 42.4 with 5 splits, key sets 49.7; at
-//   base 0 they would take 16.8 against 25.0, so a caller that knows its base
-//   passes S_kv = 1 there).
+//   base 0 they would take 16.8 against 25.0).
+// With the keys known, S_kv is cut to splits of at least kSplitKeysMin keys and
+// dropped where the launch is faster without (K/V from HBM):
+// * up to kSetsRows rows on the key sets after a prefix of at most twice the
+//   chunk (850 rows at base 1657: 36.9, 36.5 with 4 splits on 16-row tiles; at
+//   base 850 26.6 / 31.4);
+// * up to twice as many rows on the key sets with at most kSetsKeys keys: their
+//   second round of workgroups pays only there (1100 rows at base 990 37.3,
+//   42.7 with 3 splits, but 47.2 / 42.9 at base 1430; 1500 rows at base 375
+//   36.1, halves 41.1, but 59.4 / 56.8 at base 1350; 2048 rows 44.0 / 44.2 at
+//   base 0, 91.5 / 76.8 at base 2048);
+// * more rows than that after a prefix of at most twice the chunk, where two
+//   splits or none were asked for, on the halves (2000 rows at base 2600 85.4,
+//   91.7 with 2 splits). Three splits stay (1200 rows at base 1920 49.0, halves
+//   60.2).
 // Above, 32-row tiles while they give at least two workgroups per CU, and
 // 16-row tiles below that, as two halves on alternate key steps when the
 // launch has no key splits and at most two 16-row jobs per CU (the
@@ -982,9 +996,15 @@ struct PrefillChoice {
 PrefillChoice prefill_choice(uint32_t tokens, uint32_t S_kv, uint32_t keys, uint32_t cu) {
     const uint32_t ntq32 = (tokens + 31u) / 32u, ntq16 = (tokens + 15u) / 16u;
     const uint32_t jobs8 = kHkv * ((tokens + 7u) / 8u), jobs4 = kHkv * ((tokens + 3u) / 4u);
+    bool sets = S_kv == 1u && tokens <= kSetsRows;
+    if (keys != 0u) {
+        S_kv = std::min(S_kv, std::max(1u, keys / kSplitKeysMin));
+        const bool near = keys / 3u <= tokens;  // prefix of at most twice the chunk
+        sets = tokens <= kSetsRows ? near || S_kv == 1u
+                                   : tokens <= 2u * kSetsRows && keys <= kSetsKeys;
+        if (sets || (near && S_kv == 2u)) S_kv = 1u;
+    }
     const uint32_t s4 = std::min(S_kv, cu / jobs4), s8 = std::min(S_kv, cu / jobs8);
-    const bool short_prefix = keys != 0u && keys / 2u <= tokens;
-    bool sets = tokens <= (short_prefix ? 2u * kSetsRows : kSetsRows);
     if (S_kv > 1u)
         sets = tokens <= kSetsSplitRows &&
                (s8 >= std::min(S_kv, kSetsSplits) || (keys != 0u && keys <= kSetsSplitKeys * s8));

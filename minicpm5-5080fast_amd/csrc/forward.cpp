@@ -303,21 +303,6 @@ void forward_carve(Forward& f, char* p, uint32_t rows, uint32_t logit_rows) {
     f.rows = rows;
 }
 
-// Key splits of a prefill chunk's attention: none where the prefix is at most
-// twice the chunk (the unsplit key-set shapes are then the faster ones: 1024
-// rows 19.5 us against 31.0 with 2 splits; 640 rows after 1280 about equal),
-// else the reference's count for n rows (kernels.h:517-521: 4096 / n, 1..8),
-// capped so that each split gets at least kSplitKeysMin keys of the chunk's
-// last row. Splits change the result's rounding only.
-constexpr uint32_t kSplitKeysMin = 512u;
-uint32_t prefill_splits(uint32_t n, uint32_t keys) {
-    const uint32_t s = mc_kv_prefill_split_kv(n);
-    if (keys == 0u) return s;
-    if (keys / 3u <= n) return 1u;
-    const uint32_t cap = keys / kSplitKeysMin;
-    return s < cap ? s : (cap < 1u ? 1u : cap);
-}
-
 // Projections of short prefill chunks (whole model, 42 layers, best of 5;
 // library GEMMs in parentheses): 2..8 tokens through forward_prefill_rows
 // 1.74-2.16 ms (3.60-3.67), 9..32 tokens through the row GEMM 2.45-3.31 ms
@@ -347,7 +332,6 @@ mc_status_t forward_prefill_rows(const Forward& f, const int32_t* d_ids, uint32_
     const uint16_t* pending = nullptr;
     const bool step_dump = dump_due(f.dump_step);
     const bool layer_dump = step_dump && f.dump_layers;
-    const uint32_t S = prefill_splits(n, f.keys);
     FWD_OR_RETURN(mc_model_embedding_gather(w.embedding, d_ids, nullptr, cur, kHidden, n, st));
     for (uint32_t l = 0; l < kModelLayers; ++l) {
         if (layer_dump) {
@@ -362,7 +346,7 @@ mc_status_t forward_prefill_rows(const Forward& f, const int32_t* d_ids, uint32_
         FWD_OR_RETURN(mc_kv_rope_append(f.qkv, n, f.d_seq_len, l, f.d_pt, f.pool, f.layout, kTheta,
                                         rope_table_off() ? nullptr : f.inv_freq, st));
         FWD_OR_RETURN(prefill_attention(f.qkv, n, f.d_seq_len, l, f.d_pt, f.pool, f.layout, f.attn,
-                                        S > 1u ? f.pf_partials : nullptr, S, f.keys, st));
+                                        f.pf_partials, mc_kv_prefill_split_kv(n), f.keys, st));
         FWD_OR_RETURN(mc_model_gemv(w.o[l], f.attn, kHidden, f.o_out, kHidden, n, kHidden,
                                     kHidden, st));
         FWD_OR_RETURN(mc_model_gemv_resnorm_swiglu(w.gate_up[l], cur, f.o_out, w.norm2[l], other,
@@ -422,7 +406,6 @@ mc_status_t forward_prefill(const Forward& f, const int32_t* d_ids, uint32_t n, 
     const uint16_t* res_last = res + (size_t)(n - 1u) * kHidden;
     FWD_OR_RETURN(mc_model_embedding_gather(w.embedding, d_ids, nullptr, res, kHidden, n, st));
     FWD_OR_RETURN(mc_model_rmsnorm_rows(res, nullptr, w.norm1[0], f.normed, n, kHidden, kRmsEps, st));
-    const uint32_t S = prefill_splits(n, f.keys);
     // 9..32 rows: the projections through the row GEMM; larger chunks: the
     // tile GEMM
     const bool rows = n >= MC_MODEL_GEMM_ROWS_MIN && n <= MC_MODEL_GEMM_ROWS_MAX &&
@@ -471,7 +454,7 @@ mc_status_t forward_prefill(const Forward& f, const int32_t* d_ids, uint32_t n, 
                                             kTheta, inv_freq, st));
         }
         FWD_OR_RETURN(prefill_attention(f.qkv, n, f.d_seq_len, l, f.d_pt, f.pool, f.layout, f.attn,
-                                        S > 1u ? f.pf_partials : nullptr, S, f.keys, st));
+                                        f.pf_partials, mc_kv_prefill_split_kv(n), f.keys, st));
         FWD_OR_RETURN(proj_norm(f.attn, w.o[l], kHidden, f.o_out, plan.o, w.norm2[l]));
         if (layer_dump)
             FWD_OR_RETURN(dump_bf16(dump_name("layer", l, "attn_out.f32"), res_last, kHidden, st));

@@ -28,8 +28,8 @@ mc_status_t prefill_barrier_check(const char* who);
 
 
 // mc_kv_attention_prefill for a caller that knows on the host how many keys
-// the chunk's last row attends (keys; 0 = not known), which decides the
-// workgroup shape of some row counts.
+// the chunk's last row attends (keys; 0 = not known): they decide the workgroup
+// shape and how many of the S_kv splits are used.
 mc_status_t prefill_attention(const uint16_t* d_q_rows, uint32_t tokens,
                               const uint32_t* d_base_pos, uint32_t layer,
                               const uint32_t* d_page_table, const uint16_t* d_kv_pool,
