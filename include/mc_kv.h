@@ -354,7 +354,8 @@ mc_status_t mc_kv_debug_prefill_shape(uint32_t shape, uint32_t* previous);
 
 /* Key-set prefill workgroups (4 or 8 query rows, four key sets taking alternate
  * 32-key blocks): rows = 4 or 8 runs every launch on them, before the hook
- * above; 0 = chosen per launch (default). Otherwise as above. */
+ * above, unless the pool is not 16-byte aligned; 0 = chosen per launch
+ * (default). Otherwise as above. */
 mc_status_t mc_kv_debug_prefill_key_sets(uint32_t rows, uint32_t* previous);
 
 /* The workgroup shape (0..2 as above, 3 / 4: key sets of 8 / 4 rows) and key

@@ -949,7 +949,9 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(
 }
 
 // Workgroup shape and key splits of a launch of `tokens` rows with at most
-// S_kv splits on `cu` CUs; keys: those the last row attends, 0 = not known.
+// S_kv splits on `cu` CUs; keys: those the last row attends, 0 = not known;
+// sets_ok: the pool is 16-byte aligned, as the key sets' global -> LDS loads
+// need it (the tiles load K/V into registers, at any element alignment).
 // The key-set workgroups: 4 rows each while that gives every CU at most one,
 // else 8 (us per layer at base 0: 512 rows 11.0 with 4 rows, 13.2 with 8; 1024
 // rows 21.2 / 19.5).
@@ -993,20 +995,21 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(
 struct PrefillChoice {
     uint32_t shape, splits;
 };
-PrefillChoice prefill_choice(uint32_t tokens, uint32_t S_kv, uint32_t keys, uint32_t cu) {
+PrefillChoice prefill_choice(uint32_t tokens, uint32_t S_kv, uint32_t keys, uint32_t cu,
+                             bool sets_ok) {
     const uint32_t ntq32 = (tokens + 31u) / 32u, ntq16 = (tokens + 15u) / 16u;
     const uint32_t jobs8 = kHkv * ((tokens + 7u) / 8u), jobs4 = kHkv * ((tokens + 3u) / 4u);
-    bool sets = S_kv == 1u && tokens <= kSetsRows;
+    bool sets = sets_ok && S_kv == 1u && tokens <= kSetsRows;
     if (keys != 0u) {
         S_kv = std::min(S_kv, std::max(1u, keys / kSplitKeysMin));
         const bool near = keys / 3u <= tokens;  // prefix of at most twice the chunk
-        sets = tokens <= kSetsRows ? near || S_kv == 1u
-                                   : tokens <= 2u * kSetsRows && keys <= kSetsKeys;
+        sets = sets_ok && (tokens <= kSetsRows ? near || S_kv == 1u
+                                               : tokens <= 2u * kSetsRows && keys <= kSetsKeys);
         if (sets || (near && S_kv == 2u)) S_kv = 1u;
     }
     const uint32_t s4 = std::min(S_kv, cu / jobs4), s8 = std::min(S_kv, cu / jobs8);
     if (S_kv > 1u)
-        sets = tokens <= kSetsSplitRows &&
+        sets = sets_ok && tokens <= kSetsSplitRows &&
                (s8 >= std::min(S_kv, kSetsSplits) || (keys != 0u && keys <= kSetsSplitKeys * s8));
     if (sets) {
         const bool rows4 = s4 >= 1u && s4 >= s8;
@@ -1048,7 +1051,7 @@ extern "C" mc_status_t mc_kv_debug_prefill_choice(uint32_t tokens, uint32_t S_kv
         set_error("mc_kv_debug_prefill_choice: invalid args (tokens=%u S_kv=%u)", tokens, S_kv);
         return MC_E_INVALID_ARGUMENT;
     }
-    const PrefillChoice c = prefill_choice(tokens, S_kv, keys, 256u);
+    const PrefillChoice c = prefill_choice(tokens, S_kv, keys, 256u, true);
     *shape = c.shape;
     *splits = c.splits;
     return MC_OK;
@@ -1139,10 +1142,11 @@ mc_status_t prefill_attention(const uint16_t* d_q_rows, uint32_t tokens,
     const uint32_t cus = cu_count();
     const uint32_t jobs8 = kHkv * ((tokens + 7u) / 8u), jobs4 = kHkv * ((tokens + 3u) / 4u);
     uint32_t shape = g_shape.load(std::memory_order_relaxed);
-    if (const uint32_t rows = g_key_sets.load(std::memory_order_relaxed); rows != 0u)
+    const bool sets_ok = reinterpret_cast<uintptr_t>(d_kv_pool) % 16u == 0u;
+    if (const uint32_t rows = g_key_sets.load(std::memory_order_relaxed); rows != 0u && sets_ok)
         shape = rows == 4u ? kSets4 : kSets8;
     if (shape == kAutoShape) {
-        const PrefillChoice c = prefill_choice(tokens, S_kv, keys, cus ? cus : 256u);
+        const PrefillChoice c = prefill_choice(tokens, S_kv, keys, cus ? cus : 256u, sets_ok);
         shape = c.shape;
         S_kv = c.splits;
     }

@@ -48,3 +48,28 @@ def test_automatic_choice(kvm, orc, dev, T, S):
     """Either side of the row counts where the automatic choice changes; S is
     the most splits the launch may use."""
     run_prefill(kvm, orc, dev, T, 70, S, P=64, seed=T)
+
+
+class _ShiftedPool:
+    """The launcher on a copy of the pool that starts 8 bytes past a 16-byte
+    boundary."""
+
+    def __init__(self, kvm):
+        self.kvm, self.KvLayout = kvm, kvm.KvLayout
+
+    def launch_attn_prefill_flash(self, q, T, base, layer, pt, pool, *rest):
+        import torch
+        buf = torch.zeros(pool.numel() + 8, dtype=pool.dtype, device=pool.device)
+        assert buf.data_ptr() % 16 == 0
+        buf[4:4 + pool.numel()] = pool
+        self.kvm.launch_attn_prefill_flash(q, T, base, layer, pt, buf[4:4 + pool.numel()], *rest)
+        torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("T,base,S", [(33, 100, 1), (50, 300, 8)])
+def test_pool_at_an_8_byte_boundary(kvm, orc, dev, shape, T, base, S):
+    """The key sets load K/V rows straight to LDS, 16 bytes a lane; a pool
+    without that alignment runs on the tiles, forced or not."""
+    run_prefill(_ShiftedPool(kvm), orc, dev, T, base, S, P=64, seed=T)
+    kvm.debug_prefill_key_sets(0)
+    run_prefill(_ShiftedPool(kvm), orc, dev, T, base, S, P=64, seed=T)
