@@ -157,14 +157,19 @@ void launch_cfg(const RowsArgs& a, hipStream_t st) {
 // where it has several, which then cover each other's latency (SwiGLU, 32
 // rows: N = 6144 14.3 us with one stage, 15.0 with two; N = 2560 plain: 7.99
 // with one, 5.96 with four; N = 512 SwiGLU, 9 rows: 7.35 with one, the kernel
-// before 6.87). 8 waves were no faster anywhere.
+// before 6.87). SwiGLU above 8192 columns streams from HBM for so long that
+// bytes in flight count more than workgroups: three stages (9 / 32 rows, one
+// stage, the kernel before: N = 16384 25.4 / 33.9, 26.7 / 35.8, 26.9 / 35.1;
+// 65536 91.2 / 128, 96.0 / 131, 94.4 / 132; 130560 184 / 268, 189 / 271,
+// 180 / 257). 8 waves were no faster anywhere.
 template <uint32_t X8, bool SWI, uint32_t KC>
 void launch_rows8(const RowsArgs& a, hipStream_t st) {
     constexpr uint32_t kCus = 256u;
     if constexpr (SWI) {
         if (a.N <= 8u * kCus) launch_cfg<X8, 2, true, KC, 4, 4>(a, st);
         else if (a.N <= 16u * kCus) launch_cfg<X8, 2, true, KC, 4, 2>(a, st);
-        else launch_cfg<X8, 2, true, KC, 4, 1>(a, st);
+        else if (a.N <= 32u * kCus) launch_cfg<X8, 2, true, KC, 4, 1>(a, st);
+        else launch_cfg<X8, 2, true, KC, 4, 3>(a, st);
     } else {
         if (a.N <= 8u * kCus) launch_cfg<X8, 1, false, KC, 4, 4>(a, st);
         else if (a.N <= 16u * kCus) launch_cfg<X8, 2, false, KC, 4, 4>(a, st);

@@ -19,7 +19,8 @@ def P(t):
 @pytest.mark.parametrize("N,K,swi", [(16, 2048, 0), (2048, 2048, 0), (2064, 2048, 0),
                                      (4096, 2048, 0), (4112, 2048, 0), (48, 6144, 0),
                                      (2064, 6144, 0), (4112, 6144, 0), (16, 2048, 1),
-                                     (2048, 2048, 1), (2064, 2048, 1), (4112, 2048, 1)])
+                                     (2048, 2048, 1), (2064, 2048, 1), (4112, 2048, 1),
+                                     (8208, 2048, 1)])
 def test_row_groups_and_stage_counts(pkg, orc, dev, N, K, swi):
     import torch
     lib = pkg._native.lib()
