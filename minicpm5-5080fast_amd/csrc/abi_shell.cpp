@@ -219,7 +219,7 @@ struct SessionImpl {
     Breakdown bd;
     // with weights
     Forward fwd;
-    void* blas = nullptr;  // prefill GEMM library (prefill_blas_create)
+    void* blas = nullptr;  // prefill GEMM library (prefill_blas_create), mostly unused
     int32_t* h_emit = nullptr;  // pinned: the token a decode returns
 };
 
@@ -547,11 +547,11 @@ mc_status_t mc_session_create(mc_model_t model, mc_session_t* out_session) {
     s->max_chunks = mc_kv_decode_max_chunks(m->max_ctx, s->chunk_pos);
     s->act_rows = std::min(m->max_ctx, prefill_chunk_tokens());
     const size_t pool_b = (size_t)mc_kv_total_elems(s->layout) * 2u;
-    // With weights: the rocBLAS handle of the prefill projections (used when an
-    // environment variable asks for it) gets its device workspace from the
-    // arena, so it does not allocate after create.
+    // With weights and where an environment variable sends prefill projections
+    // to rocBLAS: its handle gets its device workspace from the arena, so it does
+    // not allocate after create.
     size_t blas_ws = 0;
-    if (m->weights) {
+    if (m->weights && prefill_blas_wanted()) {
         const mc_status_t bs = prefill_blas_create(&s->blas, &blas_ws);
         if (bs != MC_OK) {
             release_session(s);
@@ -619,9 +619,9 @@ mc_status_t mc_session_create(mc_model_t model, mc_session_t* out_session) {
         f.pf_partials = s->pf_partials;
         f.max_chunks = s->max_chunks;
         f.chunk_pos = s->chunk_pos;
-        rs = prefill_blas_workspace(s->blas, bufs[11], blas_ws);
+        f.blas = s->blas;
+        if (s->blas != nullptr) rs = prefill_blas_workspace(s->blas, bufs[11], blas_ws);
         if (rs == MC_OK) {
-            f.blas = s->blas;
             e = hipHostMalloc((void**)&s->h_emit, sizeof(int32_t));
             if (e != hipSuccess) rs = check_hip(e, "mc_session_create: pinned token buffer");
         }

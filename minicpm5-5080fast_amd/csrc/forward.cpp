@@ -78,6 +78,13 @@ bool gemm_defaults_only() {
     return on;
 }
 
+// MC_PREFILL_ROWS_GEMV_OFF=1 (read once per process): chunks of 2..32 tokens go
+// through rocBLAS as well.
+bool prefill_rows_gemv_off() {
+    static const bool off = std::getenv("MC_PREFILL_ROWS_GEMV_OFF") != nullptr;
+    return off;
+}
+
 // The prefill projections' GEMM library of one session.
 struct PrefillBlas {
     rocblas_handle rb = nullptr;
@@ -87,6 +94,10 @@ struct PrefillBlas {
 // W^T(N x K) . x^T(K x M)).
 mc_status_t gemm_bf16(const Forward& f, const uint16_t* x, uint32_t M, const uint16_t* W,
                       uint32_t N, uint32_t K, uint16_t* y) {
+    if (f.blas == nullptr) {
+        set_error("prefill GEMM (%u x %u x %u): the session has no rocBLAS handle", M, N, K);
+        return MC_E_INTERNAL;
+    }
     rocblas_handle h = static_cast<const PrefillBlas*>(f.blas)->rb;
     if (rocblas_set_stream(h, f.st) != rocblas_status_success) {
         set_error("prefill GEMM: rocblas_set_stream failed");
@@ -232,6 +243,8 @@ bool dump_due(uint32_t step) {
     return c.on && (int64_t)step < (int64_t)c.steps;
 }
 
+bool prefill_blas_wanted() { return gemm_defaults_only() || prefill_rows_gemv_off(); }
+
 mc_status_t prefill_blas_create(void** out, size_t* ws_bytes) {
     *out = nullptr;
     *ws_bytes = kBlasWorkspace;
@@ -303,16 +316,6 @@ void forward_carve(Forward& f, char* p, uint32_t rows, uint32_t logit_rows) {
     f.rows = rows;
 }
 
-// Projections of short prefill chunks (whole model, 42 layers, best of 5;
-// library GEMMs in parentheses): 2..8 tokens through forward_prefill_rows
-// 1.74-2.16 ms (3.60-3.67), 9..32 tokens through the row GEMM 2.45-3.31 ms
-// (3.30-3.74). MC_PREFILL_ROWS_GEMV_OFF=1 sends chunks of 2..32 tokens
-// through rocBLAS as well (the measured A/B).
-bool prefill_rows_gemv_off() {
-    static const bool off = std::getenv("MC_PREFILL_ROWS_GEMV_OFF") != nullptr;
-    return off;
-}
-
 // A prefill chunk of 2..MC_MODEL_GEMV_MAX_ROWS tokens: the projections as
 // M-row GEMVs (each weight byte read once for all rows, the residual add +
 // RMSNorm as their prologue, the SwiGLU as the gate_up epilogue; the batch
@@ -320,7 +323,9 @@ bool prefill_rows_gemv_off() {
 // path, the lm_head on the last row. The same forward as the GEMM path up to
 // the projections' fp32 summation order (reference: forward.cpp:200-420
 // runs every T > 1 chunk through its GEMMs). The residual is kept as
-// cur + pending as in forward_decode.
+// cur + pending as in forward_decode. Whole model, 42 layers: 2..8 tokens
+// 1.58-1.93 ms; 9..32 tokens through the row GEMM 1.92-2.39 ms, 33 through the
+// tile GEMM 2.15; all of them 3.3-3.7 through library GEMMs.
 mc_status_t forward_prefill_rows(const Forward& f, const int32_t* d_ids, uint32_t n,
                                  int32_t* d_next) {
     TraceRange trace_range("forward_prefill_rows");

@@ -67,7 +67,7 @@ namespace mckv {
 struct Forward {
     const ModelWeights* w = nullptr;
     hipStream_t st = nullptr;
-    void* blas = nullptr;  // prefill GEMM library (prefill_blas_create)
+    void* blas = nullptr;  // prefill GEMM library, or none (prefill_blas_wanted)
     // KV cache of a session (prefill and solo decode)
     uint16_t* pool = nullptr;
     const uint32_t* d_pt = nullptr;
@@ -106,6 +106,10 @@ bool dump_due(uint32_t step);
 size_t forward_act_bytes(uint32_t rows, uint32_t logit_rows);
 void forward_carve(Forward& f, char* base, uint32_t rows, uint32_t logit_rows);
 
+// Whether an environment variable sends some prefill projections to rocBLAS
+// (MC_PREFILL_GEMM_DEFAULT, MC_PREFILL_ROWS_GEMV_OFF; read once per process).
+// Only then does a session hold the library state below.
+bool prefill_blas_wanted();
 // GEMM library state of a session's prefill projections (a rocBLAS handle)
 // and the size of the device workspace it is to be given (*ws_bytes);
 // prefill_blas_workspace then hands it that much caller memory (carved from

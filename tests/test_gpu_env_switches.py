@@ -12,6 +12,9 @@ environment, each case in a child process of its own:
   prefill forward, 8448..65535; a prompt is prefilled in chunks of that
   size (bit-identical to mc_prefill calls of the chunk lengths), and an
   invalid value keeps 8448 with a warning.
+* MC_PREFILL_GEMM_DEFAULT, MC_PREFILL_ROWS_GEMV_OFF (no reference
+  counterpart): a session holds a rocBLAS handle and its 32 MiB workspace
+  only where one of them sends projections there.
 """
 import json
 import os
@@ -147,3 +150,35 @@ def test_prefill_chunk_from_environment(model_dir, value, cut):
     res = json.loads(r.stdout.strip().splitlines()[-1])
     assert res[cut], res
     assert ("MC_PREFILL_CHUNK" in r.stderr) == (value == "100")
+
+
+CHILD_BLAS = r"""
+import importlib, json, sys
+sys.path.insert(0, sys.argv[1])
+rt = importlib.import_module("minicpm5-5080fast_amd.runtime")
+m = rt.Model(sys.argv[2], rt.model_options(max_context_tokens=2048, max_sessions=1))
+s = rt.Session(m)
+for n in (5, 20, 48):
+    s.reset()
+    s.prefill([7 * i + 1 for i in range(n)])
+print(json.dumps(s.arena_bytes()))
+s.close()
+m.close()
+"""
+
+
+def test_blas_workspace_only_where_asked_for(model_dir):
+    path, _ = model_dir
+    names = ("MC_PREFILL_GEMM_DEFAULT", "MC_PREFILL_ROWS_GEMV_OFF")
+    got = {}
+    for name in (None,) + names:
+        e = {k: v for k, v in os.environ.items() if k not in SWITCHES + names}
+        if name is not None:
+            e[name] = "1"
+        print("child session arena", name, flush=True)
+        r = subprocess.run([sys.executable, "-c", CHILD_BLAS, ROOT, path], env=e,
+                           capture_output=True, text=True, timeout=100)
+        assert r.returncode == 0, r.stderr[-2000:]
+        got[name] = json.loads(r.stdout.strip().splitlines()[-1])
+    for name in names:
+        assert got[name] - got[None] == 32 << 20, got

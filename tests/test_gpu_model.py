@@ -845,10 +845,12 @@ def test_model_chunked_prefill_equals_split_calls(rt, model_dir):
 
 
 def test_model_prefill_allocates_nothing_after_create(rt, model_dir):
-    """The session's rocBLAS handle works in a workspace carved from the
-    session arena at create (sized by rocBLAS's own query), so prefills of
-    any length, decodes and resets leave the device's free memory unchanged
-    (memory_arena.h:1-8: no allocation after steady state)."""
+    """Everything a session needs is carved from its arena at create, so
+    prefills of any length (row GEMVs, row GEMM, tile GEMM, two chunks),
+    decodes and resets leave the device's free memory unchanged
+    (memory_arena.h:1-8: no allocation after steady state). The HIP runtime
+    loads a kernel's code at its first launch in a process; the tests above
+    have launched all of these."""
     import ctypes as C
     hip = C.CDLL("libamdhip64.so")
     hip.hipMemGetInfo.argtypes = [C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]
