@@ -125,6 +125,15 @@ mc_status_t mc_model_gemm_tiles(const uint16_t* d_w, const uint16_t* d_x, uint16
                                 float* d_partials, uint32_t M, uint32_t N, uint32_t K,
                                 uint32_t swiglu, uint32_t splits, uint32_t shape, void* stream);
 
+/* How MC_MODEL_GEMM_TILES_AUTO runs a size: rows 0..plan[0] - 1 on tile shape
+ * plan[1] in plan[3] K splits, the rest (plan[0] < M) on shape plan[2] in a
+ * second launch. form: 0 plain, 1 swiglu, 2 rope (N = 2560). N, K as above;
+ * min_splits <= max_splits <= 8, both 1 with form 1 or 2. Host only; for tests
+ * that need a size of two launches. No reference counterpart. */
+mc_status_t mc_model_debug_gemm_tiles_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t form,
+                                           uint32_t min_splits, uint32_t max_splits,
+                                           uint32_t plan[4]);
+
 /* The qkv projection of a prefill chunk with RoPE and the K/V append as its
  * epilogue, on the same tiles: rows d_x [M][K], weights d_w [2560][K]; the
  * rotated q heads go to d_qkv [M][2560], rotated k and v to the pages of

@@ -92,6 +92,8 @@ _SIGS = {
     "mc_model_gemm_tiles": (C.c_int, [_P, _P, _P, _P, _u32, _u32, _u32, _u32, _u32, _u32, _P]),
     "mc_model_gemm_tiles_rope": (C.c_int, [_P, _P, _P, _u32, _u32, _P, _u32, _P, _P, LayoutT,
                                            _u32, _P]),
+    "mc_model_debug_gemm_tiles_plan": (C.c_int, [_u32, _u32, _u32, _u32, _u32, _u32,
+                                                 C.POINTER(_u32)]),
     "mc_model_rmsnorm_splits": (C.c_int, [_P, _P, _u32, _P, _P, _u32, C.c_float, _P]),
     "mc_model_gemm_rows": (C.c_int, [_P, _P, _u32, _P, _u32, _u32, _u32, _u32, _u32, _P]),
     "mc_model_gemv_resnorm": (C.c_int, [_P, _P, _P, _P, _P, _u32, _P, _u32, _u32, _u32,

@@ -632,3 +632,22 @@ extern "C" mc_status_t mc_model_gemm_tiles_rope(const uint16_t* d_w, const uint1
     return gemm_tiles({d_x, d_w, d_qkv, nullptr, M, kRow, K, false, rope}, p,
                       (hipStream_t)stream);
 }
+
+extern "C" mc_status_t mc_model_debug_gemm_tiles_plan(uint32_t M, uint32_t N, uint32_t K,
+                                                      uint32_t form, uint32_t min_splits,
+                                                      uint32_t max_splits, uint32_t plan[4]) {
+    if (plan == nullptr || M == 0u || M > 65535u || N == 0u || N > 65536u || N % 64u != 0u ||
+        K == 0u || K > 16384u || form > 2u || (form == 2u && N != kRow) || min_splits < 1u ||
+        min_splits > max_splits || max_splits > 8u || (form != 0u && max_splits > 1u) ||
+        K % (128u * min_splits) != 0u) {
+        set_error("mc_model_debug_gemm_tiles_plan: invalid args (M=%u N=%u K=%u form=%u "
+                  "splits=%u..%u)", M, N, K, form, min_splits, max_splits);
+        return MC_E_INVALID_ARGUMENT;
+    }
+    const GemmPlan p = gemm_tiles_plan(M, N, K, (TileEnd)form, min_splits, max_splits);
+    plan[0] = p.rows0;
+    plan[1] = p.shape0;
+    plan[2] = p.shape1;
+    plan[3] = p.splits;
+    return MC_OK;
+}

@@ -99,11 +99,28 @@ def test_every_tile_shape_at_its_edges(lib, orc, dev, shape):
     (33, 2560, 2048, 0, 1, 0), (201, 2048, 2048, 0, 2, 1), (48, 2048, 6144, 0, 8, 1),
     (300, 2560, 2048, 0, 1, 0), (100, 6144, 2048, 1, 1, 0), (511, 2048, 6144, 0, 4, 1),
     (1025, 6144, 2048, 1, 1, 0), (2065, 2048, 256, 0, 1, 1),
-    (8455, 2048, 256, 0, 1, 0)])
+    (8455, 2048, 256, 0, 1, 0), (20011, 2048, 128, 0, 1, 0), (65535, 64, 128, 0, 1, 0)])
 def test_planned_shape(lib, orc, dev, M, N, K, swi, splits, part):
     """The shape the plan takes for the model's projections, more than one
-    round of workgroups, two-launch plans (8455 rows) and ragged row counts."""
+    round of workgroups, ragged row counts and the largest chunk."""
     err, guard = run(lib, orc, dev, M, N, K, swi, splits, AUTO, part, M)
+    assert err <= 1.0 and guard, (err, guard)
+
+
+def second_launch_rows(lib, M, N, K, form):
+    """Rows that the plan of least estimated time leaves to its second launch."""
+    p = (C.c_uint32 * 4)()
+    assert lib.mc_model_debug_gemm_tiles_plan(M, N, K, form, 1, 1, p) == 0
+    return M - p[0]
+
+
+@pytest.mark.parametrize("M,N,K,swi,part", [(8455, 2048, 2048, 0, 0), (8455, 2048, 2048, 0, 1),
+                                            (1300, 6144, 2048, 1, 0), (8448, 1536, 256, 1, 0)])
+def test_two_launches(lib, orc, dev, M, N, K, swi, part):
+    """Sizes that the plan cuts into whole rounds of a large tile and the rows
+    left over: the second launch's rows and outputs follow the first's."""
+    assert second_launch_rows(lib, M, N, K, swi) > 0
+    err, guard = run(lib, orc, dev, M, N, K, swi, 1, AUTO, part, M)
     assert err <= 1.0 and guard, (err, guard)
 
 
@@ -143,14 +160,30 @@ def test_norm_of_split_sums(lib, orc, dev, splits):
 def test_rope_form(lib, pkg, orc, dev, shape):
     """mc_model_gemm_tiles_rope equals the plain tiles followed by
     mc_kv_rope_append bit for bit (q columns and every page slot), for whole
-    and part tiles, both page sizes around a tile's rows and a two-launch plan."""
+    and part tiles, page sizes below and above a tile's rows and, planned, several
+    rounds of workgroups."""
+    check_rope_form(lib, pkg, orc, dev, shape, 256)
+
+
+@pytest.mark.parametrize("M,K", [(6500, 2048), (7936, 2048), (13100, 256)])
+def test_rope_form_in_two_launches(lib, pkg, orc, dev, M, K):
+    """Sizes whose qkv projection the plan cuts in two: the second launch's rows
+    are rotated and appended at their own positions."""
+    assert second_launch_rows(lib, M, 2560, K, 2) > 0
+    check_rope_form(lib, pkg, orc, dev, AUTO, K, ((M, 41, 32),))
+
+
+def check_rope_form(lib, pkg, orc, dev, shape, K, sizes=None):
     import torch
-    K, N, layer = 256, 2560, 1
+    N, layer = 2560, 1
     bm = SHAPES[shape][0] if shape != AUTO else 0
     rng = np.random.default_rng(7)
-    w = to_dev(orc.f32_to_bf16(rng.standard_normal((N, K), dtype=np.float32) / 16), dev)
-    for M, base, page in (((1, 0, 32), (bm + 1, 3001, 16), (2 * bm + 17, 77, 64)) if bm else
-                          ((33, 5, 1), (300, 900, 32), (8455, 40, 32))):
+    w = to_dev(orc.f32_to_bf16(rng.standard_normal((N, K), dtype=np.float32) /
+                               np.float32(K ** 0.5)), dev)
+    if sizes is None:
+        sizes = (((1, 0, 32), (bm + 1, 3001, 16), (2 * bm + 17, 77, 64)) if bm else
+                 ((33, 5, 1), (300, 900, 32), (8455, 40, 32)))
+    for M, base, page in sizes:
         npage = (base + M + page - 1) // page + 2
         pt = to_dev(rng.permutation(npage).astype(np.uint32), dev)
         x = to_dev(orc.f32_to_bf16(rng.standard_normal((M, K), dtype=np.float32)), dev)
