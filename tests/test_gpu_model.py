@@ -629,22 +629,22 @@ m.close()
 """
 
 
-def test_model_tuned_gemm_solutions_match_default(rt, model_dir, tmp_path):
-    """The prefill projections' tuned rocBLAS solutions (prefill_gemm_table.h)
-    against rocBLAS's default heuristic (MC_PREFILL_GEMM_DEFAULT=1, read once,
-    so in a child process): the last-row logits of prefills whose row counts
-    select tuned rows (300 rows: the 256-row gate_up row; 6200 rows: the
-    6144-row gate_up row; 8448 rows, one full chunk: gate_up and down) agree
-    to the logits tolerance (only the GEMMs' summation order differs), and
-    each prefill repeated on the same session gives bitwise the same logits."""
+def test_model_tile_gemm_matches_library(rt, model_dir, tmp_path):
+    """The prefill projections on the tile GEMM against rocBLAS
+    (MC_PREFILL_GEMM_DEFAULT=1, read once, so in a child process): the last-row
+    logits of prefills whose row counts differ in plan (33: the fewest rows;
+    201: o and down with K splits; 300; 6200; 6500: qkv in two launches; 8448:
+    one full chunk, gate_up, o and down in two) agree to the logits tolerance
+    (only the GEMMs' summation order differs), and each prefill repeated on the
+    same session gives bitwise the same logits."""
     import json
     import subprocess
     import sys
     path, _ = model_dir
-    sizes = [300, 6200, 8448]
+    sizes = [33, 201, 300, 6200, 6500, 8448]
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     out = {}
-    for tag, extra in (("tuned", {}), ("default", {"MC_PREFILL_GEMM_DEFAULT": "1"})):
+    for tag, extra in (("tiles", {}), ("library", {"MC_PREFILL_GEMM_DEFAULT": "1"})):
         env = {k: v for k, v in os.environ.items() if k != "MC_PREFILL_GEMM_DEFAULT"}
         env.update(extra)
         f = str(tmp_path / f"{tag}.npy")
@@ -652,11 +652,11 @@ def test_model_tuned_gemm_solutions_match_default(rt, model_dir, tmp_path):
                            env=env, capture_output=True, text=True, timeout=600)
         assert r.returncode == 0, r.stderr[-3000:]
         out[tag] = np.load(f)
-    for tag in out:  # deterministic GEMM solutions: a repeated prefill is bitwise equal
+    for tag in out:  # sums in a fixed order: a repeated prefill is bitwise equal
         for i, n in enumerate(sizes):
             assert np.array_equal(out[tag][2 * i], out[tag][2 * i + 1]), (tag, n)
     for i, n in enumerate(sizes):
-        rel, cos = compare_logits(out["tuned"][2 * i], out["default"][2 * i])
+        rel, cos = compare_logits(out["tiles"][2 * i], out["library"][2 * i])
         print("rows", n, "rel", rel, "cos", cos)
         assert rel < 2e-2 and cos > 0.999, n
 
@@ -682,13 +682,11 @@ m.close()
 def test_model_short_prefill_rows_path(rt, orc, model_dir, tmp_path):
     """Prefill chunks of 2..8 tokens run their projections as M-row GEMVs
     (forward_prefill_rows), chunks of 9..32 tokens through the row GEMM
-    (mc_model_gemm_rows), and a 48-token chunk through hipBLASLt (the library
-    path of 33..1023 rows). Their last-row logits match the oracle's forward,
-    the greedy continuation matches the oracle's decode, and they agree with
-    the library GEMM path (MC_PREFILL_ROWS_GEMV_OFF=1, read once, so in a
-    child process) to the logits tolerance. The child imports no torch and so
-    runs /opt/rocm's rocBLAS / hipBLASLt, where this process runs PyTorch's;
-    the 48-token chunk differs between the two only in rounding. A prompt
+    (mc_model_gemm_rows), and a 48-token chunk through the tile GEMM. Their
+    last-row logits match the oracle's forward, the greedy continuation matches
+    the oracle's decode, and they agree with rocBLAS for all projections
+    (MC_PREFILL_ROWS_GEMV_OFF=1 for 2..32 tokens and MC_PREFILL_GEMM_DEFAULT=1
+    above, read once, so in a child process) to the logits tolerance. A prompt
     prefilled as a 20-token
     call (row GEMM) and a 5-token call (row GEMVs) gives the same logits on
     two sessions and matches the oracle."""
@@ -725,7 +723,7 @@ def test_model_short_prefill_rows_path(rt, orc, model_dir, tmp_path):
     s.close()
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     f = str(tmp_path / "gemm.npy")
-    env = dict(os.environ, MC_PREFILL_ROWS_GEMV_OFF="1")
+    env = dict(os.environ, MC_PREFILL_ROWS_GEMV_OFF="1", MC_PREFILL_GEMM_DEFAULT="1")
     r = subprocess.run([sys.executable, "-c", _ROWS_CHILD, root, path, f, json.dumps(prompts)],
                        env=env, capture_output=True, text=True, timeout=600)
     assert r.returncode == 0, r.stderr[-3000:]
@@ -749,6 +747,28 @@ def test_model_short_prefill_rows_path(rt, orc, model_dir, tmp_path):
     assert rel < 2e-2 and cos > 0.999, (rel, cos)
     a.close()
     b.close()
+    m.close()
+
+
+@pytest.mark.parametrize("base,n", [(900, 850), (2200, 1100), (2048, 2048), (3001, 777),
+                                    (12000, 300)])
+def test_model_follow_up_chunk(rt, model_dir, base, n):
+    """A chunk after a prefix, whose attention shape and key splits follow from
+    both (key sets, halves, 16-row tiles with splits), gives the logits of the
+    same prompt prefilled at once, to the logits tolerance."""
+    path, _ = model_dir
+    m = rt.Model(path, rt.model_options(max_context_tokens=16384, max_sessions=1))
+    s = rt.Session(m)
+    p = [(i * 7919 + 5) % 130560 for i in range(base + n)]
+    s.prefill(p)
+    whole = s.last_logits()
+    s.reset()
+    s.prefill(p[:base])
+    s.prefill(p[base:])
+    rel, cos = compare_logits(s.last_logits(), whole)
+    print(base, n, "rel", rel, "cos", cos)
+    assert rel < 2e-2 and cos > 0.999, (rel, cos)
+    s.close()
     m.close()
 
 

@@ -24,6 +24,13 @@ def test_tile_and_block_edges(kvm, orc, dev, shape, T, base):
         run_prefill(kvm, orc, dev, T, base, 1, P=P, seed=T + base)
 
 
+@pytest.mark.parametrize("T,base", [(1100, 60), (1500, 300), (2048, 100)])
+def test_two_rounds_of_workgroups(kvm, orc, dev, shape, T, base):
+    """1025 to 2048 rows, which a session runs on 8-row workgroups where the
+    prefix is short: more workgroups than CUs, the heaviest tiles first."""
+    run_prefill(kvm, orc, dev, T, base, 1, seed=T)
+
+
 @pytest.mark.parametrize("S", [2, 3, 8])
 def test_splits(kvm, orc, dev, shape, S):
     """Key splits, some of them without keys (40 keys over 8 splits)."""
