@@ -595,13 +595,13 @@ def bench_model(pkg, torch, steps):
         cfg = rt.gen_config(max_new_tokens=1 << 20)
         prompt = [(i * 7919) % W.VOCAB for i in range(2048)]
         s = rt.Session(m)
-        s.prefill(prompt)  # first use: rocBLAS loads its GEMM kernels
+        s.prefill(prompt)  # first use: the runtime loads the kernels' code
         s.reset()
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         s.prefill(prompt)
         prefill_s = time.perf_counter() - t0
-        # short prompts (projections as row-group GEMVs up to 16 tokens)
+        # short prompts (8: row GEMVs, 16 and 32: row GEMM)
         short = {}
         for n in (8, 16, 32):
             s.reset()

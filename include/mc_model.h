@@ -10,8 +10,8 @@
  * arguments, MC_E_CUDA for launch failures, message in mc_last_error().
  *
  * mc_model_load (minicpm_runtime.h) uses these when the model directory holds
- * model.wpk: prefill runs the GEMMs through rocBLAS (bf16 in/out, fp32
- * compute), decode and batch steps run the GEMV kernels below.
+ * model.wpk: prefill chunks run the GEMV kernels (2..8 tokens), the row GEMM
+ * (9..32) and the tile GEMM below, decode and batch steps the GEMV kernels.
  */
 #ifndef MC_MODEL_H_
 #define MC_MODEL_H_
@@ -114,11 +114,11 @@ mc_status_t mc_model_gemm_rows(const uint16_t* d_w, const uint16_t* d_x, uint32_
  * rounded to bf16, as mc_model_gemm_rows. With d_partials instead of d_y the
  * fp32 sums of each of `splits` equal K ranges go to d_partials[split][M][N]
  * (splits > 1 needs it; not with swiglu). Rows are contiguous (strides K and
- * N), N a multiple of 64, K of 128 * splits, pointers 16-byte aligned. shape: MC_MODEL_GEMM_TILES_AUTO (least estimated
- * time) or a row 0..MC_MODEL_GEMM_TILES_SHAPES - 1 of the tile table
- * (MC_E_INVALID_ARGUMENT where it does not take the sizes). No reference
- * counterpart: the reference runs multi-token chunks through cuBLAS
- * (forward.cpp:200-420). */
+ * N), N a multiple of 64, K of 128 * splits, pointers 16-byte aligned. shape:
+ * MC_MODEL_GEMM_TILES_AUTO (least estimated time) or a row
+ * 0..MC_MODEL_GEMM_TILES_SHAPES - 1 of the tile table (MC_E_INVALID_ARGUMENT
+ * where it does not take the sizes). No reference counterpart: the reference
+ * runs multi-token chunks through cuBLAS (forward.cpp:200-420). */
 #define MC_MODEL_GEMM_TILES_SHAPES 18u
 #define MC_MODEL_GEMM_TILES_AUTO 0xFFFFFFFFu
 mc_status_t mc_model_gemm_tiles(const uint16_t* d_w, const uint16_t* d_x, uint16_t* d_y,

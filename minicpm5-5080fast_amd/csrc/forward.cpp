@@ -12,10 +12,11 @@
 //   and logits are bf16.
 //
 // MI355X mapping:
-//   * prefill (T rows): projections through the row GEMM (9..32 rows), the
-//     tile GEMM (gemm_tiles.hip; the SwiGLU as gate_up's epilogue, K splits of
-//     o and down summed by the norm that follows); RMSNorm / residual-add
-//     kernels, the paged prefill attention; the lm_head of the last row
+//   * prefill (T rows): projections through the GEMVs (2..8 rows), the row GEMM
+//     (9..32) or the tile GEMM (gemm_tiles.hip; RoPE and the K/V append as qkv's
+//     epilogue, the SwiGLU as gate_up's, K splits of o and down summed by the
+//     norm that follows); RMSNorm / residual-add kernels, the paged prefill
+//     attention; the lm_head of the last row
 //     through the GEMV. rocBLAS runs them only when an environment variable
 //     asks for it (MC_PREFILL_GEMM_DEFAULT, MC_PREFILL_ROWS_GEMV_OFF);
 //   * decode (one row) and batch steps (n <= 8 rows): every projection is the

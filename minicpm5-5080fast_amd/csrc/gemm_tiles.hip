@@ -24,9 +24,13 @@
 // 34.6 -> 31 us per 32-step round against issuing the loads in one burst.
 //
 // What bounds it: up to ~500 rows the bytes a CU pulls through its L1 (x and
-// W tiles, about 50-80 B/ns per CU with W coming from HBM), so the tile and
-// split are chosen to give every CU one workgroup; above, the MFMA rate
-// (256 x 256 tiles at 8448 rows: 1.15 PFLOP/s with the SwiGLU included).
+// W tiles, about 50-80 B/ns per CU) and W's arrival from HBM (gate_up at 201
+// rows: 22.1 us, 18.2 with W in cache), so the tile and split are chosen to
+// give every CU one workgroup; above, the load stream and the MFMAs together,
+// which overlap only in part (gate_up at 2048 rows, timing-only variants: 123
+// us whole, 87 without loads, 71 with MFMAs alone, 81 without MFMAs; MFMA busy
+// 57% of CU cycles there, 66% in the 256 x 256 tiles at 8448 rows, which reach
+// 1.15 PFLOP/s with the SwiGLU included).
 // The four projections of a layer, weights from HBM (graph replay; the library
 // GEMMs that ran before and the separate SwiGLU kernel in parentheses): 64
 // rows 34 us (71), 201 rows 51 (82), 512 rows 74 (97), 1024 rows 119 (139),
@@ -380,8 +384,12 @@ void launch_tile(const GemmTiles& g, uint32_t splits, hipStream_t st) {
 // step grows with BM + BN, the bytes a K step brings in, so a larger tile does
 // more per byte but leaves CUs idle when the shape gives it few tiles or a
 // short last round: the plan takes the shapes and split of least estimated
-// time (on the measured tables 1.5% above the best choice on average, 15% at
-// worst).
+// time (on the measured tables of the plain and SwiGLU forms 1.5% above the best
+// choice on average, 15% at worst). The RoPE form has no fit of its own: it is
+// planned with the plain form's costs, which are 7-20% under its launches (30.3
+// us for 25.9 estimated at 2048 rows, 88 for 76 at 8448) but order the shapes
+// alike: over 29 row counts from 33 to 8448 the planned launch is within 2% of
+// the best single shape.
 struct TileCost {
     float launch, round, step;  // step 0: the shape does not take this form
 };

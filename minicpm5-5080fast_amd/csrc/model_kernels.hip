@@ -413,8 +413,10 @@ __global__ void __launch_bounds__(64u * WV)
 
     // The row is streamed in groups of kG chunks per lane (K / (512 kG) groups
     // per row); the next group's loads (of this row or the next one) are
-    // issued before the current group is multiplied, so each lane keeps 2 kG
-    // 16-byte loads in flight whatever K is. The first group is requested
+    // issued before the current group is multiplied. They are conditional, so
+    // the compiler's wait counts after the join assume that they were not
+    // issued (vmcnt 3 to 0 for the current group's four): each group in effect
+    // waits for the next one's loads as well. The first group is requested
     // before the activation prologue: the weights do not depend on it, so the
     // two memory latencies overlap instead of adding up.
     // one activation row: the whole weight row is requested at once (12
